@@ -330,7 +330,7 @@ def _plan_kernel_ms(f, call, reps=5):
 
 def _config1(args):
     """relu(matmul(x, w)) in float32, x [256, 512], w [512, 1024]: the reference's bit-exact float32 fold
-    (gemm_exact, VALU)."""
+    (gemm_fold, VALU)."""
     import numpy as np
 
     import lumen_amd as L
@@ -351,7 +351,7 @@ def _config1(args):
     k_ms = per[dom]
     roof = {"bound": "valu", "achieved": round(flops / (k_ms * 1e-3) / 1e12, 3), "peak": 157.3, "unit": "TFLOP/s",
             "frac": round(flops / (k_ms * 1e-3) / 1e12 / 157.3, 4), "traffic": None,
-            "kernel": f"{f.plan.steps[dom].kind} step {dom}: gemm_exact relu(matmul) f32 (sequential-k fold)",
+            "kernel": f"{f.plan.steps[dom].kind} step {dom}: gemm_fold relu(matmul) f32 (sequential-k fold)",
             "per_launch": {"flops": flops, "bytes": 3670016, "ms": round(k_ms, 4)}}
     cpu = None
     if not args.no_cpu:

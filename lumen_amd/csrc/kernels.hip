@@ -3,6 +3,7 @@
 #include <cstring>
 
 #include "gemm.h"
+#include "gemm_fold.h"
 #include "nhip_internal.h"
 
 using namespace nhipk;
@@ -78,6 +79,39 @@ int default_config(const nhip_gemm_desc *d) {
         if (tiles >= 256) return c;
     }
     return kNumTiled - 1;
+}
+
+// Rows a wave of gemm_fold takes: as many, up to 4, as leave 2048 waves (two a SIMD, one's reads under the
+// other's sums). Measured with 1 / 2 / 4 / 8 rows: [256, 512] x [512, 1024] 18.3 / 14.1 / 17.7 / 34.4 us, 1024^3
+// 98.9 / 69.2 / 58.8 / 75.2, [512, 100] x [100, 2000] 17.3 / 12.8 / 10.2 / 11.0, [64, 500] x [500, 1000] 9.3 /
+// 11.4 / 17.8 / 32.0. A contiguous along m takes a scalar load a k, which more rows share: up to 8, and 1024
+// waves suffice (512^3 52.1 / 32.1 / 26.6 / 35.9 us, 2048^3 2790 / 1429 / 749 / 440).
+int fold_rows(const nhip_gemm_desc *d) {
+    const int64_t columns = (d->n + 63) / 64 * batch_count(d), waves = d->a_k == 1 ? 2048 : 1024;
+    for (int rm = d->a_k == 1 ? 4 : 8; rm > 1; rm /= 2)
+        if (d->m >= rm && (d->m + rm - 1) / rm * columns >= waves) return rm;
+    return 1;
+}
+
+template <int RM, bool AK, bool BN>
+int launch_fold_rows(hipStream_t st, GemmShape s, const nhip_gemm_desc *d, const float *a, const float *b, void *out) {
+    s.tiles_m = int((s.m + 4 * RM - 1) / (4 * RM));
+    s.tiles_n = int((s.n + 63) / 64);
+    dim3 grid(s.tiles_m * s.tiles_n, unsigned(batch_count(d)));
+    hipLaunchKernelGGL((gemm_fold<RM, AK, BN, AnyStore>), grid, dim3(256), 0, st, s, a, b, AnyStore{out, d->d_dtype});
+    return check(hipGetLastError(), "gemm_fold launch");
+}
+
+template <bool AK, bool BN>
+int launch_fold(hipStream_t st, const GemmShape &s, const nhip_gemm_desc *d, const float *a, const float *b, void *out) {
+    switch (fold_rows(d)) {
+        case 8:
+            if constexpr (!AK) return launch_fold_rows<8, AK, BN>(st, s, d, a, b, out);
+            [[fallthrough]];
+        case 4: return launch_fold_rows<4, AK, BN>(st, s, d, a, b, out);
+        case 2: return launch_fold_rows<2, AK, BN>(st, s, d, a, b, out);
+        default: return launch_fold_rows<1, AK, BN>(st, s, d, a, b, out);
+    }
 }
 
 template <typename TD>
@@ -350,6 +384,15 @@ int gemm_on(hipStream_t st, const nhip_gemm_desc *d, const void *a, const void *
             return fail("nhip_gemm: the streamed configs need k to be a multiple of their k tile");
         if (d->a_dtype == NHIP_F16) return launch_mfma<true>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
         return launch_mfma<false>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
+    }
+    // float32 with each operand contiguous along one axis; other strides, and 16-bit operands in no MFMA layout,
+    // go through gemm_exact
+    if (d->a_dtype == NHIP_F32 && d->k > 0 && d->k < (int64_t(1) << 30) && (d->a_k == 1 || d->a_m == 1) &&
+        (d->b_k == 1 || d->b_n == 1)) {
+        const float *fa = static_cast<const float *>(a), *fb = static_cast<const float *>(b);
+        if (d->a_k == 1)
+            return d->b_n == 1 ? launch_fold<true, true>(st, s, d, fa, fb, out) : launch_fold<true, false>(st, s, d, fa, fb, out);
+        return d->b_n == 1 ? launch_fold<false, true>(st, s, d, fa, fb, out) : launch_fold<false, false>(st, s, d, fa, fb, out);
     }
     switch (d->d_dtype) {
         case NHIP_F32: return launch_exact<float>(st, s, d, a, b, out);

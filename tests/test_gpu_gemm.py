@@ -215,3 +215,37 @@ def test_gemm_persistent_f16_operands(hip):
     nv.call("nhip_gemm", C.byref(desc), da.ptr, db.ptr, dd.ptr)
     got = dd.get((m, n), np.float32)
     assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max() + 1e-4
+
+
+@pytest.mark.parametrize("at,bt", [(False, True), (False, False), (True, True), (True, False)])
+@pytest.mark.parametrize("m,n,k,z,out", [
+    (1, 1, 1, 1, nv.NHIP_F32), (3, 65, 31, 1, nv.NHIP_F32), (5, 130, 32, 2, nv.NHIP_F32), (17, 64, 33, 1, nv.NHIP_BF16),
+    (250, 1029, 97, 1, nv.NHIP_F32), (37, 300, 160, 3, nv.NHIP_F16), (515, 520, 71, 1, nv.NHIP_F32),
+    (1030, 1000, 40, 1, nv.NHIP_F32)])
+def test_float32_fold_is_bit_exact_in_every_layout(hip, at, bt, m, n, k, z, out):
+    """float32 dots against the sequential fold (a rounded product added to a rounded sum, k in order), bit for
+    bit: 1, 2, 4 and 8 rows a wave, ragged rows, columns and k, batches, every memory order. An infinity and a
+    NaN stay in their row, and a fold that ends in -0 keeps its sign."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((z, m, k)).astype(np.float32)
+    b = rng.standard_normal((z, k, n)).astype(np.float32)
+    if m > 4:
+        a[0, 1], a[0, 3, -1], a[0, 4, 0] = -0.0, np.inf, np.nan
+    want = np.zeros((z, m, n), np.float32)
+    with np.errstate(invalid="ignore"):
+        for i in range(k):
+            want += a[:, :, i, None] * b[:, None, i, :]
+    da = Dev(np.ascontiguousarray(a.transpose(0, 2, 1)) if at else a)
+    db = Dev(b if bt else np.ascontiguousarray(b.transpose(0, 2, 1)))
+    dd = Dev(nbytes=z * m * n * 4)
+    desc = _desc(m, n, k, 1 if at else k, m if at else 1, n if bt else 1, 1 if bt else k, dt=nv.NHIP_F32, out=out,
+                 batch=(z,), sa=(m * k,), sb=(k * n,), sd=(m * n,))
+    nv.call("nhip_gemm", C.byref(desc), da.ptr, db.ptr, dd.ptr)
+    if out == nv.NHIP_F32:
+        np.testing.assert_array_equal(dd.get((z, m, n), np.float32), want)
+    else:
+        got = dd.get((z, m, n), np.uint16)
+        with np.errstate(over="ignore", invalid="ignore"):
+            bits = D.bf16_bits(want) if out == nv.NHIP_BF16 else want.astype(np.float16).view(np.uint16)
+        ok = ~np.isnan(want)
+        assert np.array_equal(got[ok], bits[ok]) and ok.sum() >= (m - 1) * n
