@@ -163,6 +163,12 @@ typedef struct {
 /* O = softmax(scale Q K^T [causal]) V, P rounded to the inputs' dtype before P V; writes LSE = m + log l
  * (kernel.py:99-102). */
 int nhip_flash_fwd(const nhip_attn_desc *desc, const void *q, const void *k, const void *v, void *o, float *lse);
+/* The same with `workspace` of nhip_flash_fwd_workspace bytes. Where few query rows meet many keys (config -1) the
+ * keys are divided over waves, and with a workspace (null: without) over workgroups too, whose float32 partial sums
+ * it holds until a second kernel adds them in order. */
+int nhip_flash_fwd_ws(const nhip_attn_desc *desc, const void *q, const void *k, const void *v, void *o, float *lse,
+                      void *workspace);
+int nhip_flash_fwd_workspace(const nhip_attn_desc *desc, size_t *bytes);
 /* Number of forward tile configs nhip_attn_desc.config accepts (0: 128 queries a workgroup, the default for -1;
  * 1: 256; 2: 64) for autotuning and forced configs (the CUDA attention `Config`,
  * lumen/codegen/attention/cuda/mod.rs:312-420). */
@@ -237,7 +243,7 @@ typedef struct {
 
 enum {
     NHIP_STEP_GEMM = 1,       /* desc: nhip_gemm_desc; pointers: a, b, d (and the workspace when splits > 1) */
-    NHIP_STEP_FLASH_FWD = 2,  /* desc: nhip_attn_desc; pointers: q, k, v, o, lse */
+    NHIP_STEP_FLASH_FWD = 2,  /* desc: nhip_attn_desc; pointers: q, k, v, o, lse (and the workspace, or none) */
     NHIP_STEP_FLASH_BWD = 3,  /* desc: nhip_attn_desc; pointers: q, k, v, o, do, lse, dq, dk, dv, ws */
     NHIP_STEP_COPY = 4,       /* desc: uint64 bytes; pointers: dst, src */
     NHIP_STEP_FILL = 5,       /* desc: uint64 bytes, uint32 byte value; pointers: dst */

@@ -15,6 +15,8 @@ casts -- becomes one ``flash_attention_backward`` fusion producing dQ, dK and dV
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 
 from lumen_amd.graph.ir import Graph, Node, TensorType
@@ -578,11 +580,12 @@ def lower(plan, step):
         a.v_b, a.v_n, a.v_s = vl.strides[vb[0]], vl.strides[vb[1]], vl.strides[vs]
         ol = loc[step.outputs[0]]  # [B, N, Sq, D]
         a.o_b, a.o_n, a.o_s = ol.strides[0], ol.strides[1], ol.strides[2]
-        if len(step.outputs) > 1:
-            lse = loc[step.outputs[1]]
-        else:
-            lse = plan.scratch[id(step)]
-        return nv.NHIP_STEP_FLASH_FWD, a, [ql, kl, vl, ol, lse]
+        scratch, lse_bytes = plan.scratch.get(id(step)), forward_lse_bytes(g, step.outputs)
+        lse = loc[step.outputs[1]] if len(step.outputs) > 1 else scratch
+        ops = [ql, kl, vl, ol, lse]
+        if step.scratch > lse_bytes:  # the workspace follows
+            ops.append(dataclasses.replace(scratch, offset=scratch.offset + lse_bytes // 4))
+        return nv.NHIP_STEP_FLASH_FWD, a, ops
     q, k, v, o, do, lse = n.inputs
     qt, kt = g.types[q], g.types[k]
     ls = {x: loc[x] for x in (q, k, v, o, do, lse)}
@@ -604,6 +607,32 @@ def lower(plan, step):
         setattr(a, f"{name}_n", l_.strides[2])
     ws = plan.scratch[id(step)]
     return nv.NHIP_STEP_FLASH_BWD, a, [ls[q], ls[k], ls[v], ls[o], ls[do], ls[lse], outs[0], outs[1], outs[2], ws]
+
+
+def forward_lse_bytes(g, outputs) -> int:
+    """Scratch bytes for a forward's LSE when no other step reads it (a multiple of 256)."""
+    if len(outputs) > 1:
+        return 0
+    t = g.types[outputs[0]]
+    return -(-t.numel() // t.shape[-1] * 4 // 256) * 256
+
+
+def forward_workspace_bytes(g, node) -> int:
+    """Workspace bytes of nhip_flash_fwd_ws for a forward node, as the library itself reports them."""
+    import ctypes as C
+
+    from lumen_amd import native as nv
+
+    p = node.params
+    q, k, v = (g.types[u] for u in node.inputs)
+    (qb, qs, qd), (kb, ks, _), (_, _, vd) = p["q_dims"], p["k_dims"], p["v_dims"]
+    a = nv.AttnDesc()
+    a.batch, a.heads, a.kv_heads = q.shape[qb[0]], q.shape[qb[1]], k.shape[kb[1]]
+    a.sq, a.sk, a.head_dim, a.value_head_dim = q.shape[qs], k.shape[ks], q.shape[qd], v.shape[vd]
+    a.dtype, a.causal, a.config = (1 if q.dtype == "bfloat16" else 2), int(p["causal"]), -1
+    n = C.c_size_t()
+    nv.call("nhip_flash_fwd_workspace", C.byref(a), C.byref(n))
+    return n.value
 
 
 def _need_unit(*pairs):

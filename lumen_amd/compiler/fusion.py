@@ -275,8 +275,10 @@ def fuse(graph: Graph, fuse_loops=True, packed=frozenset()) -> list:
                     st.mode = backward_mode(b, nh, sq, sk)
                     hdv = graph.types[node.inputs[2]].shape[3]
                     st.scratch = backward_workspace_bytes(b, nh, sq, sk, hd, kvh, st.mode, hdv)
-                elif len(outs) == 1:
-                    st.scratch = graph.types[outs[0]].numel() // graph.types[outs[0]].shape[-1] * 4
+                else:
+                    from lumen_amd.compiler.attention import forward_lse_bytes, forward_workspace_bytes
+
+                    st.scratch = forward_lse_bytes(graph, outs) + forward_workspace_bytes(graph, node)
         elif kinds[k] in ("view", "reduce"):
             st = Step(kinds[k], nodes, outs)
         else:

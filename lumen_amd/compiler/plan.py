@@ -1032,7 +1032,7 @@ class Plan:
     ATTN_AUTOTUNE_FLOPS = 1 << 32  # flash forwards of fewer FLOPs keep the default tile
 
     def _autotune_attention(self, workspace_ptr, input_ptrs):
-        """Times each forward tile config on a flash forward step's own operands (HIP events, 3 runs after a
+        """Times the default and each forward tile config on a flash forward step's own operands (HIP events, 3 runs after a
         warm-up) and keeps the fastest (a later one must win by ``AUTOTUNE_MARGIN``); picks are shared by
         steps of the same shape, layout and dtype."""
         from lumen_amd import native as nv
@@ -1054,13 +1054,15 @@ class Plan:
                 for loc in ops:
                     base = workspace_ptr if loc.base[0] == "ws" else input_ptrs[loc.base[1]]
                     ptrs.append(base + loc.offset * D.size_of(loc.dtype))
-                best, best_ms = 0, float("inf")
-                for cfg in range(n_cfg.value):
+                # the library's own choice first, which may divide the keys (through the step's workspace)
+                ptrs += [None] * (6 - len(ptrs))
+                best, best_ms = -1, float("inf")
+                for cfg in range(-1, n_cfg.value):
                     desc.config = cfg
-                    nv.call("nhip_flash_fwd", C.byref(desc), *ptrs)  # warm-up
+                    nv.call("nhip_flash_fwd_ws", C.byref(desc), *ptrs)  # warm-up
                     ev0.record()
                     for _ in range(3):
-                        nv.call("nhip_flash_fwd", C.byref(desc), *ptrs)
+                        nv.call("nhip_flash_fwd_ws", C.byref(desc), *ptrs)
                     ev1.record()
                     ms = ev0.elapsed_ms(ev1) / 3
                     if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):

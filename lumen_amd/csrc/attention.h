@@ -1205,8 +1205,13 @@ int launch_fwd(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *
     }
 }
 
+// Whether a forward divides the keys over waves (attention_split.h), and that launch: `ws` as
+// flash_fwd_workspace_bytes says, or null for one workgroup a row tile.
+bool split_keys(const nhip_attn_desc *d);
+int launch_split(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *d, void *ws);
+
 int flash_fwd_on(hipStream_t s, const nhip_attn_desc *d, const void *q, const void *k, const void *v, void *o,
-                 float *lse) {
+                 float *lse, void *ws) {
     if (check_attn(d, "flash attention", 256)) return 1;
     if (d->sq == 0 || d->batch == 0 || d->heads == 0) return 0;
     nhipk::AttnParams p = attn_params(d);
@@ -1216,6 +1221,7 @@ int flash_fwd_on(hipStream_t s, const nhip_attn_desc *d, const void *q, const vo
     p.o = static_cast<uint16_t *>(o);
     p.lse = lse;
     bool f16 = d->dtype == NHIP_F16;
+    if (split_keys(d)) return launch_split(s, p, d, ws);
 #define NHIP_FWD(DD, FF, CC) return launch_fwd<DD, FF, CC>(s, p, d)
     const int64_t kd = kernel_dim(d);
     if (kd == 256) {

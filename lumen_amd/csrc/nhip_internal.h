@@ -20,7 +20,7 @@ hipStream_t stream_of_current();
 int gemm_on(hipStream_t s, const nhip_gemm_desc *d, const void *a, const void *b, void *out);
 int gemm_splitk_on(hipStream_t s, const nhip_gemm_desc *d, const void *a, const void *b, void *out, void *ws);
 int flash_fwd_on(hipStream_t s, const nhip_attn_desc *d, const void *q, const void *k, const void *v, void *o,
-                 float *lse);
+                 float *lse, void *ws);
 int flash_bwd_on(hipStream_t s, const nhip_attn_desc *d, const void *q, const void *k, const void *v,
                  const void *o, const void *d_o, const float *lse, void *dq, void *dk, void *dv, void *ws);
 int fill_on(hipStream_t s, void *dst, size_t bytes, unsigned char value);

@@ -609,7 +609,7 @@ static int run_steps(Plan *plan, void *workspace, void *const *inputs, size_t ni
                 break;
             case NHIP_STEP_FLASH_FWD:
                 rc = flash_fwd_on(s, reinterpret_cast<const nhip_attn_desc *>(st.args.data()), ptrs[0], ptrs[1],
-                                  ptrs[2], ptrs[3], static_cast<float *>(ptrs[4]));
+                                  ptrs[2], ptrs[3], static_cast<float *>(ptrs[4]), ptrs[5]);
                 break;
             case NHIP_STEP_FLASH_BWD:
                 rc = flash_bwd_on(s, reinterpret_cast<const nhip_attn_desc *>(st.args.data()), ptrs[0], ptrs[1],

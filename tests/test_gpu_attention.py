@@ -313,3 +313,41 @@ def test_partial_tiles_ignore_what_earlier_kernels_left_in_lds(hip, d, dv, sq, s
         for name, a, w in zip(("o", "dq", "dk", "dv"), got, want):
             assert np.isfinite(a).all(), (name, mode)
             np.testing.assert_allclose(a, w, rtol=2e-2, atol=1e-2 * max(1.0, np.abs(w).max()), err_msg=f"{name} {mode}")
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("case", [
+    (1, 1, 1, 1, 1, 64, True, 1), (2, 1, 31, 4, 2, 128, True, 2), (1, 1, 1000, 4, 4, 128, True, 1),
+    (3, 4, 517, 8, 2, 64, True, 2), (1, 33, 300, 2, 1, 128, True, 1), (2, 7, 260, 6, 1, 96, False, 1),
+    (1, 40, 40, 4, 2, 32, True, 2), (1, 100, 611, 3, 3, 64, True, 1), (1, 1, 4099, 16, 1, 40, False, 2)])
+def test_forward_with_keys_divided_over_waves(hip, case, workspace):
+    """Few query rows: O and LSE against float64 for one and several row tiles, tiles that hold rows of several
+    heads of a group, key counts around the 32-key tiles and the waves' and workgroups' shares, padded head dims;
+    with a workspace (keys split over workgroups) and without."""
+    b, sq, sk, n, nkv, d, causal, dt = case
+    rng = np.random.default_rng(sk + d)
+    np_t = np.float16
+    bits = D.bf16_bits if dt == 1 else lambda x: x.astype(np_t).view(np.uint16)
+    wide = D.bf16_to_f32 if dt == 1 else lambda x: x.view(np_t).astype(np.float32)
+    q, k, v = (bits(rng.standard_normal(s).astype(np.float32)) for s in ((b, sq, n, d), (b, sk, nkv, d), (b, sk, nkv, d)))
+    desc = attn_desc(b, sq, sk, n, nkv, d, causal, 1.0 / math.sqrt(d), dtype=dt)
+    size = C.c_size_t()
+    nv.call("nhip_flash_fwd_workspace", C.byref(desc), C.byref(size))
+    if sk > 4000:
+        assert size.value > 0  # 1 head of 4099 keys is split over workgroups
+    dq, dk, dv, o, lse = Dev(q), Dev(k), Dev(v), Dev(nbytes=q.nbytes), Dev(nbytes=b * n * sq * 4)
+    ws = Dev(nbytes=size.value)
+    nv.call("nhip_flash_fwd_ws", C.byref(desc), dq.ptr, dk.ptr, dv.ptr, o.ptr, lse.ptr, ws.ptr if workspace else None)
+    qf, kf, vf = (wide(x).astype(np.float64) for x in (q, k, v))
+    kf, vf = np.repeat(kf, n // nkv, axis=2), np.repeat(vf, n // nkv, axis=2)
+    s = np.einsum("bqnh,bknh->bnqk", qf, kf) / np.sqrt(d)
+    if causal:
+        s = np.where(np.arange(sk)[None, :] <= np.arange(sq)[:, None] + sk - sq, s, -np.inf)
+    top = s.max(-1, keepdims=True)
+    e = np.exp(s - top)
+    want = np.einsum("bnqk,bknh->bqnh", e / e.sum(-1, keepdims=True), vf)
+    got = wide(o.get((b, sq, n, d), np.uint16)).astype(np.float64)
+    tol = 2.0 ** (-8 if dt == 1 else -11)  # one rounding of P and one of O
+    assert np.abs(got - want).max() <= 4 * tol * np.abs(want).max()
+    np.testing.assert_allclose(lse.get((b, n, sq), np.float32), (top + np.log(e.sum(-1, keepdims=True)))[..., 0],
+                               rtol=0, atol=1e-4)
