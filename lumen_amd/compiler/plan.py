@@ -345,6 +345,12 @@ class Plan:
                     perm = tuple(us[0].params["permutation"])
                     if perm[-1] == len(perm) - 1:
                         o_perm[st.outputs[0]] = perm
+        # such a transpose that the graph returns is fused as a copying loop: with the operand laid out its way
+        # it is a view like any other
+        for st in self.steps:
+            if st.kind == "loop" and len(st.nodes) == 1 and st.nodes[0].prim == "transpose" \
+                    and o_perm.get(st.nodes[0].inputs[0]) == tuple(st.nodes[0].params["permutation"]):
+                st.kind = "view"
         # views first: resolved lazily in step order; a view that strides cannot express becomes a copy
         last_use: dict[int, int] = {}
         base_of: dict[int, int] = {}

@@ -537,3 +537,23 @@ def test_norm_statistics_are_read_not_stored_broadcast():
             if readers and all(k in ("loop", "row") for k in readers):  # kernels that can recompute it
                 assert not (n.prim == "cast" and src is not None and src.dtype == "bfloat16" and n.inputs[0] in
                             {o for s in p.steps for o in s.outputs}), (st.label(), v)
+
+
+def test_returned_attention_output_is_written_in_place():
+    """An attention output the graph returns is laid out as the transpose that is returned: no copying step, in a
+    forward alone and beside a backward that reads it too."""
+    import lumen_amd.functional as F
+
+    def fwd(q, k, v):
+        return F.flash_attention(q, k, v, is_causal=True)
+
+    def train(q, k, v, do):
+        o, pull = L.vjp(fwd, q, k, v)
+        return [o, *pull(do)]
+
+    for fn, n in ((fwd, 3), (train, 4)):
+        args = [L.empty((2, 96, 4, 64), "bfloat16", "meta") for _ in range(n)]
+        g = L.make_graph(fn)(*args)
+        plan = Plan(g, "hip:0", build_kernels=False)
+        assert {st.kind for st in plan.steps} <= {"flash_fwd", "flash_bwd", "view"}
+        assert plan.output_locs[0].contiguous() and plan.output_locs[0].shape == (2, 96, 4, 64)
