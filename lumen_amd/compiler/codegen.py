@@ -1150,7 +1150,8 @@ class LoopKernel:
             self.args.append(("in", v))
         for k, v in enumerate(self.step.outputs):
             ps.append(f"{STORE_T[self.graph.types[v].dtype]}*{_restrict(v, self.aliased)} out{k}")
-            self.args.append(("out", v))
+            sums = [o for _, o in self.step.colsums]  # stored a workgroup apiece in the step's scratch
+            self.args.append(("scratch", sums.index(v)) if v in sums else ("out", v))
         return ", ".join(ps)
 
     def _emitter(self, rows=None):
@@ -1271,8 +1272,9 @@ class LoopKernel:
         g, st = self.graph, self.step
         R, C = st.rows
         reds = [n for n in st.nodes if n.prim in ("reduce_sum", "reduce_max")]
+        sums = dict(st.colsums)  # value -> its column sums, an output of this kernel
         outs_elem = [v for v in st.outputs if g.types[v].numel() == R * C and R * C != R]
-        outs_row = [v for v in st.outputs if v not in outs_elem]
+        outs_row = [v for v in st.outputs if v not in outs_elem and v not in sums.values()]
         # the vector width follows the operands read or written along the columns; per-row values (a row's
         # target class, its statistics) are loaded once a row and do not narrow it
         per_row = {R, 1} if C > 1 else set()
@@ -1350,6 +1352,9 @@ class LoopKernel:
                     _declared(em).add(cidx)
                 idx = ("rc", "r", cidx, vbase(j), lane)
                 lanes.append([em.value(v, idx) for v in outs_elem])
+                for k, v in enumerate(sums):
+                    guard = "live" if exact else f"live && (({j} * {T} + tid) * {V}) < {C}LL"
+                    em.emit(f"if ({guard}) cs{k}_{j}_{lane} += {em.value(v, idx)};")
             for k, v in enumerate(outs_elem):
                 oi = st.outputs.index(v)
                 dt = g.types[v].dtype
@@ -1364,15 +1369,19 @@ class LoopKernel:
                     )
                 if not exact:
                     s = f"if ((({j} * {T} + tid) * {V}) < {C}LL) {{ {s} }}"
+                if sums:
+                    s = f"if (live) {{ {s} }}"
                 em.emit(s)  # stored as soon as computed: a chunk's results are not held across the row
         for v in outs_row:
             oi = st.outputs.index(v)
             val = em.value(v, ("r", "r"))
             dt = g.types[v].dtype
             addr = self._out_addr(self.out_views[v], g.types[v].shape, "r")
-            stores.append(f"if (tid == 0) out{oi}[{addr}] = {_store(val, dt)};")
+            stores.append(f"if (tid == 0{' && live' if sums else ''}) out{oi}[{addr}] = {_store(val, dt)};")
         body = em.lines
         pro = self._vec_prologue(em, V)
+        if sums:
+            return self._row_sums(body, pro, stores, T, J, V, R, C, sums)
         threads = T * rows_per_block
         self.grid, self.block = (-(-R // rows_per_block), 1, 1), (threads, 1, 1)
         self.lds = 0
@@ -1396,6 +1405,71 @@ class LoopKernel:
         rest = [l for l in body if l not in decl]
         src += ["  " + l for l in decl + pro + rest + stores]
         src += ["}"]
+        return "\n".join(src)
+
+    # Row kernels that sum columns: 512 threads (several rows at once) a workgroup, at most SUM_BLOCKS workgroups of at
+    # least SUM_ROWS rows a row group. Each stores its sums and a second kernel adds them: atomic adds by every
+    # workgroup to one [C] vector cost 0.19 us an add and address, one after another (a [16384, 2048] norm backward
+    # 107 us with 256 workgroups, 146 with 512, 238 with 1024; 53 with stored sums).
+    SUM_THREADS = 512
+    SUM_BLOCKS = 512
+    SUM_ROWS = 4
+
+    def _row_sums(self, body, pro, stores, T, J, V, R, C, sums):
+        """The row kernel ``body`` over many rows a workgroup, with each thread's column sums kept in registers: the
+        row groups' are added through LDS in order and stored as the workgroup's row of a ``[workgroups, C]`` scratch
+        value, which ``<name>_sum<k>`` adds up."""
+        groups = max(1, self.SUM_THREADS // T)
+        threads = groups * T
+        blocks = max(1, min(self.SUM_BLOCKS, -(-R // (groups * self.SUM_ROWS))))
+        self.grid, self.block, self.lds = (blocks, 1, 1), (threads, 1, 1), 0
+        accs = [(k, j, l) for k in range(len(sums)) for j in range(J) for l in range(V)]
+        src = [f'extern "C" __global__ __launch_bounds__({threads}) void {self.name}({self._params()}) {{',
+               f"  const int tid = threadIdx.x % {T}, group = threadIdx.x / {T}, lane = tid & 63, wave = tid >> 6;",
+               f"  __shared__ double red_lds_all[{groups}][{max(1, T // 64)}];",
+               f"  __shared__ int64_t red_ldsi_all[{groups}][{max(1, T // 64)}];",
+               "  double *red_lds = red_lds_all[group]; int64_t *red_ldsi = red_ldsi_all[group];",
+               "  (void)lane; (void)wave; (void)red_lds; (void)red_ldsi;"]
+        if groups > 1:
+            src.append(f"  __shared__ float sums_lds[{groups - 1}][{C}];")
+        src += ["  float " + ", ".join(f"cs{k}_{j}_{l} = 0" for k, j, l in accs) + ";",
+                f"  for (int64_t r0 = (int64_t)blockIdx.x * {groups}; r0 < {R}LL; r0 += {blocks * groups}LL) {{",
+                f"    const bool live = r0 + group < {R}LL;  // every thread takes part in the row reductions",
+                f"    const int64_t r = live ? r0 + group : {R - 1}LL;"]
+        decl = [l for l in body if (l.startswith("const int64_t c") or l.startswith("const int c")) and "(( " not in l]
+        src += ["    " + l for l in decl + pro + [l for l in body if l not in decl] + stores]
+        src.append("  }")
+        for k, o in enumerate(sums.values()):
+            oi = self.step.outputs.index(o)
+            at = [(j, l, f"(({j} * {T} + tid) * {V} + {l})") for j in range(J) for l in range(V)]
+            if groups > 1:
+                src += ["  __syncthreads();", "  if (group > 0) {"]
+                src += [f"    if ({c} < {C}) sums_lds[group - 1][{c}] = cs{k}_{j}_{l};" for j, l, c in at]
+                src += ["  }", "  __syncthreads();"]
+            src.append("  if (group == 0) {")
+            for j, l, c in at:
+                total = " + ".join([f"cs{k}_{j}_{l}"] + [f"sums_lds[{x}][{c}]" for x in range(groups - 1)])
+                src.append(f"    if ({c} < {C}) out{oi}[(int64_t)blockIdx.x * {C} + {c}] = {total};")
+            src.append("  }")
+        src.append("}")
+        # 16 columns x 32 row lanes a workgroup: enough workgroups, and a lane's up to 16 loads in flight at once
+        self.sum_grid, self.sum_block = (-(-C // 16), 1, 1), (512, 1, 1)
+        for k, o in enumerate(sums.values()):
+            addr = self._out_addr(self.out_views[o], self.graph.types[o].shape, "c")
+            src += [f'extern "C" __global__ __launch_bounds__(512) void {self.name}_sum{k}(const float* __restrict__ part, '
+                    "float* __restrict__ out) {",
+                    "  __shared__ float lanes[32][17];",
+                    "  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;",
+                    "  const int64_t c = (int64_t)blockIdx.x * 16 + tx;",
+                    "  float acc = 0;",
+                    f"  if (c < {C}LL)",
+                    f"    for (int r = ty; r < {blocks}; r += 32) acc += part[(int64_t)r * {C} + c];",
+                    "  lanes[ty][tx] = acc;",
+                    "  __syncthreads();",
+                    f"  if (ty == 0 && c < {C}LL) {{",
+                    "    for (int y = 1; y < 32; ++y) acc += lanes[y][tx];",
+                    f"    out[{addr}] = acc;",
+                    "  }", "}"]
         return "\n".join(src)
 
     # ---- general reductions

@@ -42,6 +42,7 @@ class Step:
     name: str = ""
     scratch: int = 0                # bytes of workspace the step needs while it runs
     mode: int | None = None         # flash_bwd: the dQ mode (nhip_attn_desc.deterministic)
+    colsums: list = field(default_factory=list)  # row: (value, its sum over the rows), the sum an output
 
     def label(self):
         return " → ".join(n.prim for n in self.nodes[:6]) + (" → …" if len(self.nodes) > 6 else "")
@@ -396,7 +397,7 @@ def _drop_unread(graph, steps):
             if len(outs) < len(st.outputs):
                 st.outputs = outs
                 by_out = {m.output: m for m in st.nodes}
-                live, stack = set(), list(outs)
+                live, stack = set(), list(outs) + [u for u, _ in st.colsums]
                 while stack:
                     v = stack.pop()
                     if v in live or v not in by_out:
@@ -537,6 +538,70 @@ def absorb_rows(graph, steps):
             break
     return [st for i, st in enumerate(steps) if i not in merged]
 
+
+def column_sums(graph, steps):
+    """Moves a float32 sum over the leading axes (a norm weight's gradient) into a row kernel that reads the same
+    rows: the kernel writing the summed ``[R, C]`` value, or one reading all that a loop computing it reads. The row
+    kernel keeps each column's sum in registers over the rows it takes (``Step.colsums``) and the value, written and
+    read back only for the sum, never exists. Values nothing reads once loops have moved are dropped too."""
+    outputs = set(graph.outputs)
+    pos, readers = {}, {}
+    for si, st in enumerate(steps):
+        for v in st.outputs:
+            pos[v] = si
+        for u in st.inputs:
+            readers.setdefault(u, []).append(st)
+    gone = set()
+    for st in steps:
+        if st.kind != "reduce" or len(st.nodes) != 1 or st.nodes[0].prim != "reduce_sum":
+            continue
+        red = st.nodes[0]
+        u, x = red.inputs[0], graph.types[red.inputs[0]]
+        if tuple(red.params["axes"]) != tuple(range(len(x.shape) - 1)) or x.dtype != "float32" \
+                or graph.types[red.output].dtype != "float32":
+            continue
+        space = (math.prod(x.shape[:-1]), x.shape[-1])
+        if space[0] < COLSUM_MIN_ROWS or u in outputs or u not in pos or readers.get(u) != [st]:
+            continue
+        made = steps[pos[u]]
+        reader = min((steps.index(r) for r in readers.get(red.output, [])), default=len(steps))
+        if made.kind == "row" and made.rows == space:
+            row = made
+        elif made.kind == "loop" and made.outputs == [u]:
+            def takes(r):
+                ri = steps.index(r)
+                have = {m.output for m in r.nodes}
+                joined = sorted(r.nodes + [m for m in made.nodes if m.output not in have], key=lambda m: m.output)
+                return (r.kind == "row" and r.rows == space and ri < reader and any(v in r.inputs for v in made.inputs)
+                        and all(v in r.inputs or pos.get(v, -1) < ri for v in made.inputs)
+                        and row_reads_ok(graph, joined, space))
+
+            row = next((r for r in steps if takes(r)), None)
+            if row is None:
+                continue
+            have = {m.output for m in row.nodes}
+            row.nodes = sorted(row.nodes + [m for m in made.nodes if m.output not in have], key=lambda m: m.output)
+            gone.add(id(made))
+        else:
+            continue
+        row.colsums = row.colsums + [(u, red.output)]
+        row.outputs = [v for v in row.outputs if v != u] + [red.output]
+        row.scratch = len(row.colsums) * colsum_bytes(space)
+        row.inputs = _inputs_of(row.nodes)
+        pos[red.output] = steps.index(row)
+        gone.add(id(st))
+    return _drop_unread(graph, [st for st in steps if id(st) not in gone])
+
+
+
+def colsum_bytes(space):
+    """Scratch bytes of one value's column sums in a row kernel: a float32 row a workgroup."""
+    from lumen_amd.compiler.codegen import LoopKernel
+
+    return min(LoopKernel.SUM_BLOCKS, -(-space[0] // LoopKernel.SUM_ROWS)) * space[1] * 4
+
+
+COLSUM_MIN_ROWS = 256  # fewer rows: not worth a kernel that adds the workgroups' sums
 
 # Horizontal fusion (``passes/horizontal.rs:40-49,79-393``): small independent loop kernels share one launch.
 HFUSE_MAX_ELEMENTS = 1 << 20      # a member's outputs are at most this many elements each

@@ -13,7 +13,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 import struct
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 from lumen_amd import dtypes as D
 from lumen_amd.compiler import attention as attn_pass
@@ -221,6 +221,7 @@ class Plan:
         if config.compiler.fuse:
             steps = fusion.hoist_to_producers(self.graph, steps)
             steps = fusion.absorb_rows(self.graph, steps)
+            steps = fusion.column_sums(self.graph, steps)
         if config.compiler.fuse and config.compiler.horizontal_fusion:
             steps = fusion.horizontal(self.graph, steps)
         return steps
@@ -825,13 +826,22 @@ class Plan:
                     relocs = (nv.Reloc * 1)(reloc(0, out))
                     call("nhip_plan_add_builtin", plan, nv.NHIP_STEP_FILL, desc, len(desc), relocs, 1)
                 relocs = []
+                def part(i):  # the i-th column sum's rows in the step's scratch
+                    loc = self.scratch[id(st)]
+                    return replace(loc, offset=loc.offset + i * fusion.colsum_bytes(st.rows) // 4)
+
                 for j, (kind, v) in enumerate(k.args):
-                    relocs.append(reloc(8 * j, self.loc[v]))
+                    relocs.append(reloc(8 * j, part(v) if kind == "scratch" else self.loc[v]))
                 args = b"\0" * (8 * len(k.args))
                 grid = (C.c_uint32 * 3)(*k.grid)
                 block = (C.c_uint32 * 3)(*k.block)
                 rr = (nv.Reloc * max(1, len(relocs)))(*relocs)
                 call("nhip_plan_add_launch", plan, fn, grid, block, k.lds, args, len(args), rr, len(relocs))
+                for i, (_, v) in enumerate(st.colsums):
+                    fn = nv.module_function(self.objects[si], f"{k.name}_sum{i}")
+                    rr = (nv.Reloc * 2)(reloc(0, part(i)), reloc(8, self.loc[v]))
+                    call("nhip_plan_add_launch", plan, fn, (C.c_uint32 * 3)(*k.sum_grid), (C.c_uint32 * 3)(*k.sum_block),
+                         0, b"\0" * 16, 16, rr, 2)
             elif st.kind == "dot":
                 desc, ops = self._gemm_desc(st.nodes[0])
                 desc.config = getattr(st, "config", -1)

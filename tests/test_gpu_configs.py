@@ -559,3 +559,32 @@ def test_gelu_gradient_closed_form_matches_float64():
     np.testing.assert_array_equal(got[n:n + 2], gd[n:n + 2])
     assert np.all(got[n + 2:n + 4] == 0.0), got[n + 2:n + 4]
     assert np.all(np.isnan(got[n + 4:])), got[n + 4:]
+
+
+@pytest.mark.parametrize("rows,cols", [(256, 64), (257, 72), (1000, 100), (700, 520), (3001, 2048), (300, 8192), (259, 1111)])
+def test_norm_backward_row_kernel_sums_its_weight_gradient(hip, rows, cols):
+    """RMS norm forward and backward in float32 as one row kernel with the weight's gradient summed over the rows it
+    takes (one and several rows at a time, ragged row counts and row widths), against float64: the sum within the
+    rounding of its float32 additions."""
+    rng = np.random.default_rng(rows + cols)
+    x, dy = (rng.standard_normal((rows, cols)).astype(np.float32) for _ in range(2))
+    w = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+
+    def train(x, w, dy):
+        y, pull = L.vjp(lambda x, w: F.rms_norm(x, x.size(-1), w), x, w)
+        return [y, *pull(dy)]
+
+    f = L.compile(train, device="hip")
+    args = [L.from_numpy(a).to("hip") for a in (x, w, dy)]
+    for _ in range(2):  # the second call adds into sums the first one left
+        y, dx, dw = (L.to_numpy(t) for t in f(*args))
+    assert any(st.colsums for st in f.plan.steps)
+    x6, w6, g6 = x.astype(np.float64), w.astype(np.float64), dy.astype(np.float64)
+    inv = 1 / np.sqrt((x6 * x6).mean(1, keepdims=True) + 2.0**-23)
+    d = g6 * w6
+    terms = g6 * inv * x6
+    np.testing.assert_allclose(y, x6 * inv * w6, rtol=1e-5, atol=1e-6)
+    want = d * inv - x6 * (d * x6).mean(1, keepdims=True) * inv**3
+    assert np.abs(dx - want).max() <= 1e-5 * np.abs(want).max()
+    bound = (rows + 8) * 2.0**-24 * np.abs(terms).sum(0)
+    assert np.all(np.abs(dw - terms.sum(0)) <= bound)

@@ -557,3 +557,22 @@ def test_returned_attention_output_is_written_in_place():
         plan = Plan(g, "hip:0", build_kernels=False)
         assert {st.kind for st in plan.steps} <= {"flash_fwd", "flash_bwd", "view"}
         assert plan.output_locs[0].contiguous() and plan.output_locs[0].shape == (2, 96, 4, 64)
+
+
+def test_norm_weight_gradient_sums_join_the_row_kernel():
+    """A norm's backward over enough rows is one row kernel that also sums the weight's gradient: no [R, C] value is
+    stored for the sum, in a norm alone and in a block; few rows keep the separate reduction."""
+    def train(x, w, dy):
+        y, pull = L.vjp(lambda x, w: F.rms_norm(x.float(), x.size(-1), w.float()).bfloat16(), x, w)
+        return [y, *pull(dy)]
+
+    p = _plan(train, ((512, 256), "bfloat16"), ((256,), "bfloat16"), ((512, 256), "bfloat16"))
+    rows = [st for st in p.steps if st.kind == "row"]
+    assert [st.kind for st in p.steps] == ["row", "loop"] and len(rows[0].colsums) == 1
+    assert sorted(p.graph.types[v].shape for v in rows[0].outputs) == [(256,), (512, 256), (512, 256)]
+    p = _plan(train, ((64, 256), "bfloat16"), ((256,), "bfloat16"), ((64, 256), "bfloat16"))
+    assert "reduce" in [st.kind for st in p.steps]
+    model, opt = W.build(W.TINY)
+    ids = L.empty([W.TINY.batch, W.TINY.seq], "int64", "meta")
+    p = Plan(trace(W.train_step, (model, opt, ids, ids)).graph, build_kernels=False)
+    assert sum(len(st.colsums) for st in p.steps) >= 2
