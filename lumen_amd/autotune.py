@@ -119,4 +119,6 @@ def forced(cls):
 
 def forced_key() -> tuple:
     """The effective forced configs, for plan cache keys."""
+    if not _FORCED:
+        return ()
     return tuple(c.key() for c in (forced(HipGemmConfig), forced(HipAttentionConfig)) if c is not None)

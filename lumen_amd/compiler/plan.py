@@ -16,6 +16,7 @@ import struct
 from dataclasses import dataclass, replace
 
 from lumen_amd import dtypes as D
+from lumen_amd import native as nv
 from lumen_amd.compiler import attention as attn_pass
 from lumen_amd.compiler import codegen, fusion, kcache, merge, passes, remat, schedule
 from lumen_amd.config import config
@@ -1161,15 +1162,14 @@ class Plan:
     def run_in(self, workspace_ptr: int, input_ptrs: list):
         """Queues the plan on the stream: inputs are device pointers in graph-input order. The first run
         autotunes the plan's large GEMMs on its own buffers (when ``config.compiler.autotune``)."""
-        from lumen_amd import native as nv
-
         if self._native is None:
             self._apply_forced()
             if config.compiler.autotune:
                 self._autotune(workspace_ptr, input_ptrs)
-        plan = self._native_plan()
-        arr = (C.c_void_p * max(1, len(input_ptrs)))(*input_ptrs)
-        nv.call("nhip_plan_run", plan, C.c_void_p(workspace_ptr), arr, len(input_ptrs))
+            self._native_plan()
+        if nv.lib().nhip_plan_run(self._native, workspace_ptr, (C.c_void_p * max(1, len(input_ptrs)))(*input_ptrs),
+                                  len(input_ptrs)):
+            raise RuntimeError(nv.lib().nhip_last_error().decode())
 
     def capture(self, workspace_ptr: int, input_ptrs: list):
         """A HIP graph of one whole run bound to these pointers (``nhip_plan_capture``); launch it with

@@ -62,7 +62,10 @@ class CompilerFlags:
     def key(self):
         from lumen_amd import autotune
 
-        flags = tuple((f.name, getattr(self, f.name)) for f in dataclasses.fields(self) if f.name != "_version")
+        version, flags = self.__dict__.get("_flags", (None, None))
+        if version != self._version:  # setting any flag moves the version on
+            flags = tuple((f.name, getattr(self, f.name)) for f in dataclasses.fields(self) if f.name != "_version")
+            self.__dict__["_flags"] = (self._version, flags)
         return flags + (("forced", autotune.forced_key()),)
 
 

@@ -14,9 +14,11 @@ import functools
 
 import numpy as np
 
+from lumen_amd import dtypes as D
 from lumen_amd import nn
 from lumen_amd.config import config
 from lumen_amd.graph.trace import trace, tree_leaves
+from lumen_amd.graph.tracer import TracedTensor
 from lumen_amd import native
 from lumen_amd.tensor import DeviceBuffer, Tensor, device_name, device_type, empty
 
@@ -71,7 +73,7 @@ class Compiled:
                     w._placed(target)
                 for pack in plan.packs:
                     _pack([traced.weights[traced.layout[i][1]] for i in pack], target)
-            entry = (traced, plan, workspace)
+            entry = (traced, plan, workspace, plan and _Recipe(traced, plan))
             self._plans[key] = entry
         self._latest = key
         return target, entry
@@ -117,8 +119,8 @@ class Compiled:
         plan are kept, so alternating inputs replay too). Profiled runs (``plan.profile``) and plans of fewer
         than GRAPH_MIN_STEPS native steps are never captured.
         Returns the input pointers the run read."""
-        short = len(getattr(plan, "native_steps", ())) < self.GRAPH_MIN_STEPS and plan._native is not None
-        if not config.compiler.hip_graphs or getattr(plan, "_profiling", False) or short:
+        short = plan._native is not None and len(plan.native_steps) < self.GRAPH_MIN_STEPS
+        if short or not config.compiler.hip_graphs or getattr(plan, "_profiling", False):
             plan.run_in(workspace.ptr, ptrs)
             return ptrs
         graphs = self._graphs.get(id(plan))
@@ -160,49 +162,52 @@ class Compiled:
         return self._plans[self._latest][0].graph
 
     def __call__(self, *args):
-        target, (traced, plan, workspace) = self._prepare(args)
-        g = traced.graph
+        target, (traced, plan, workspace, recipe) = self._prepare(args)
         ran = plan is not None and not any(isinstance(a, Tensor) and device_type(a.device) == "meta" for a in args)
         if not ran:
+            g = traced.graph
             outs = [Tensor(g.types[v].dtype, g.types[v].shape, "meta") for v in g.outputs]
         else:
             keep = []
-            ptrs = []
-            tensors = [a for a in args if isinstance(a, Tensor)]
-            scalars = _scalars(args)
+            if recipe.args:
+                tensors = [a for a in args if isinstance(a, Tensor)]
+            if recipe.scalars:
+                scalars = _scalars(args)
             for kind, k in traced.layout:
                 if kind == "arg":
                     t = tensors[k]
-                    if device_name(t.device) != target:
+                    if t.device != target:
                         t = t.to(device=target)
-                    keep.append(t)
-                    ptrs.append(t.data_ptr())
                 elif kind == "scalar":
                     t = self._device_scalar(target, scalars[k])
-                    keep.append(t)
-                    ptrs.append(t.data_ptr())
                 else:
                     t = traced.weights[k]._placed(target)
-                    keep.append(t)
-                    ptrs.append(t.data_ptr())
-            ptrs = self._run(plan, workspace, traced, ptrs, keep)
+                keep.append(t)
+            ptrs = self._run(plan, workspace, traced, [t.data_ptr() for t in keep], keep)
             self._last_buffers = (workspace.ptr, ptrs)
-            outs = []
-            for v, loc in zip(g.outputs, plan.output_locs):
-                if loc.base[0] == "in":  # computed over the weight it replaces
-                    outs.append(keep[loc.base[1]])
-                    continue
-                t = Tensor(loc.dtype, loc.shape, target, buffer=workspace, offset=loc.offset * _size(loc.dtype))
-                outs.append(t)
+            # outputs computed over the weight they replace, or views of the workspace
+            outs = [keep[i] if i is not None else Tensor.on_device(dtype, shape, target, workspace, offset)
+                    for i, dtype, shape, offset in recipe.outputs]
             # the other weights the function assigned: written back into their memory, in stream order
-            for j, k in enumerate(traced.written):
-                if traced.n_returned + j not in plan.in_place_outputs:
-                    traced.weights[k]._placed(target).copy_(outs[traced.n_returned + j])
+            for j, k in recipe.copied_back:
+                traced.weights[k]._placed(target).copy_(outs[j])
             self._keep = keep
         for i, path, value in traced.static_writes:
             nn.assign(args[i], path, value)
-        it = iter(outs)
-        return _rebuild(traced.out, it)
+        return _rebuild(traced.out, iter(outs))
+
+
+class _Recipe:
+    """What a call of a plan does, worked out once: which kinds of inputs its layout names, where each output lies
+    (``(input position or None, dtype, shape, byte offset in the workspace)``) and the weights copied back."""
+
+    def __init__(self, traced, plan):
+        kinds = {kind for kind, _ in traced.layout}
+        self.args, self.scalars = "arg" in kinds, "scalar" in kinds
+        self.outputs = [(loc.base[1] if loc.base[0] == "in" else None, loc.dtype, tuple(loc.shape),
+                         loc.offset * _size(loc.dtype)) for loc in plan.output_locs]
+        self.copied_back = [(traced.n_returned + j, k) for j, k in enumerate(traced.written)
+                            if traced.n_returned + j not in plan.in_place_outputs]
 
 
 def _pack(weights, target):
@@ -229,16 +234,10 @@ def _pack(weights, target):
 
 
 def _size(dtype):
-    from lumen_amd import dtypes as D
-
     return D.size_of(dtype)
 
 
 def _scalars(args):
-    out = []
-    for a in args:
-        if isinstance(a, float):
-            out.append(a)
     # module floats follow the top-level ones in trace order
     res = []
     for a in args:
@@ -251,8 +250,6 @@ def _scalars(args):
 
 
 def _rebuild(out, it):
-    from lumen_amd.graph.tracer import TracedTensor
-
     if isinstance(out, TracedTensor):
         return next(it)
     if isinstance(out, (list, tuple)):

@@ -8,6 +8,7 @@ taking it compiles, its data written there by ``copy_`` / ``load_state_dict``.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import numpy as np
@@ -16,18 +17,22 @@ from lumen_amd import dtypes as D
 from lumen_amd import native
 
 
-def device_name(d) -> str:
-    """``"hip:0"`` from ``"hip"``, ``"hip:0"``, ``"cpu"``, ``"meta"``. The GPU device is named ``hip``; there is
-    no CUDA alias."""
-    d = str(d)
+@functools.lru_cache(maxsize=256)
+def _device_name(d: str) -> str:
     kind, _, idx = d.partition(":")
     if kind not in ("cpu", "hip", "meta"):
         raise ValueError(f"unknown device {d!r}: this backend has cpu (host data), hip and meta")
     return f"{kind}:{idx or 0}"
 
 
+def device_name(d) -> str:
+    """``"hip:0"`` from ``"hip"``, ``"hip:0"``, ``"cpu"``, ``"meta"``. The GPU device is named ``hip``; there is
+    no CUDA alias."""
+    return _device_name(str(d))
+
+
 def device_type(d) -> str:
-    return device_name(d).split(":")[0]
+    return device_name(d).partition(":")[0]
 
 
 def device_index(d) -> int:
@@ -76,6 +81,15 @@ class Tensor:
         self._placements = {}
         self._pending = None
         self.grad = None
+
+    @classmethod
+    def on_device(cls, dtype, shape, device, buffer, offset):
+        """A device tensor over ``buffer`` whose canonical dtype, shape tuple and device name the caller has."""
+        t = cls.__new__(cls)
+        t.dtype, t.shape, t.device = dtype, shape, device
+        t._host, t._buffer, t._offset = None, buffer, offset
+        t._is_parameter, t._placements, t._pending, t.grad = False, {}, None, None
+        return t
 
     # -- basics
     @property
