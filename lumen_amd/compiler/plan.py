@@ -58,6 +58,12 @@ def _mfma_layout(d) -> bool:
     return all(d.a_batch[i] % 8 == 0 and d.b_batch[i] % 8 == 0 for i in range(d.nbatch))
 
 
+def _skinny(d) -> bool:
+    """Whether a dot in an MFMA layout runs as few rows by default: kernels.hip's skinny_default."""
+    groups = 1 if d.m <= 16 else 2 if d.m <= 32 else 4
+    return d.m <= 64 and d.a_k == 1 and d.b_k == 1 and groups * d.n <= 24576 and (groups <= 2 or d.k <= 2048)
+
+
 def _contig(shape):
     return codegen._contig(shape)
 
@@ -1146,6 +1152,8 @@ class Plan:
         except NotImplementedError:
             return 1, None
         if not _mfma_layout(d) or any((loc.offset * D.size_of(loc.dtype)) % 16 for loc in (lhs, rhs)):
+            return 1, None
+        if _skinny(d):
             return 1, None
         z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
         tiles = -(-d.m // 256) * -(-d.n // 256) * z

@@ -4,6 +4,7 @@
 
 #include "gemm.h"
 #include "gemm_fold.h"
+#include "gemm_skinny.h"
 #include "nhip_internal.h"
 
 using namespace nhipk;
@@ -36,8 +37,8 @@ constexpr int kNumTiled = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kStream4w = kNumTiled, kStream8w = kNumTiled + 1, kStream8w32 = kNumTiled + 2,
               kStream128 = kNumTiled + 3, kStreamPersist = kNumTiled + 4, kStream8wX = kNumTiled + 5,
               kStream8wP = kNumTiled + 6, kStream4wX = kNumTiled + 7, kStream4w64X = kNumTiled + 8,
-              kStream8w64X = kNumTiled + 9;
-constexpr int kNumConfigs = kNumTiled + 10;
+              kStream8w64X = kNumTiled + 9, kSkinny = kNumTiled + 10;
+constexpr int kNumConfigs = kNumTiled + 11;
 
 GemmShape shape_of(const nhip_gemm_desc *d) {
     GemmShape s;
@@ -67,11 +68,29 @@ int64_t batch_count(const nhip_gemm_desc *d) {
     return z;
 }
 
+constexpr int64_t kSkinnyRows = 64;
+
+bool skinny_ok(const nhip_gemm_desc *d) {
+    return d->m <= kSkinnyRows && d->a_k == 1 && d->b_k == 1 && d->k < (int64_t(1) << 30);
+}
+
+// Whether gemm_skinny is the default (plan.py's _skinny is the same rule). Every workgroup reads A's rows (in whole 16s,
+// 64 above 32) once, so many columns or many rows of a long k make those reads the larger part. Measured, us of
+// this and of the 128 x 128 kernel at its best split: [16, 2048] x [8192, 2048] 9.7, 17.4; [16, 8192] x [2048, 8192]
+// 16.4, 19.0; [16, 4096] x [1024, 4096] 9.5, 17.1; [32, 8192] x [2048, 8192] 23.7, 27.5; [64, 2048] x [4096, 2048]
+// 11.7, 18.2. Not: [16, 2048] x [32000, 2048] 37.4, 31.7; [64, 2048] x [8192, 2048] 20.6, 19.4; [64, 8192] x
+// [2048, 8192] 37.5, 19.8; [35, 3648] x [14592, 3648] 56.8, 51.7.
+bool skinny_default(const nhip_gemm_desc *d) {
+    const int64_t groups = d->m <= 16 ? 1 : d->m <= 32 ? 2 : 4;
+    return skinny_ok(d) && groups * d->n <= 24576 && (groups <= 2 || d->k <= 2048);
+}
+
 // The default tile for a shape: the streamed 256 x 256 kernel when k allows it and its tiles fill the 256 CUs,
 // else the streamed 128 x 128 kernel (two workgroups a CU) when its tiles fill half of them, else the largest
 // tiled config whose tile count fills them at least once.
 int default_config(const nhip_gemm_desc *d) {
     int64_t z = batch_count(d);
+    if (skinny_default(d)) return kSkinny;
     if (d->k % 64 == 0 && ((d->m + 255) / 256) * ((d->n + 255) / 256) * z >= 256) return kStream8w;
     if (d->k % 64 == 0 && ((d->m + 127) / 128) * ((d->n + 127) / 128) * z >= 128) return kStream128;
     for (int c = 0; c < kNumTiled; ++c) {
@@ -262,6 +281,28 @@ int launch_stream_persist(hipStream_t st, GemmShape s, int64_t z, const void *a,
 }
 
 
+template <bool F16, int MT, int NW>
+int launch_skinny_waves(hipStream_t st, const GemmShape &s, int64_t z, const void *a, const void *b, void *out, int dtype) {
+    hipLaunchKernelGGL((gemm_skinny<F16, MT, NW>), dim3(unsigned((s.n + 15) / 16), unsigned(z)), dim3(64 * NW), 0, st, s,
+                       static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(b), AnyStore{out, dtype});
+    return check(hipGetLastError(), "gemm_skinny launch");
+}
+
+// 16 waves a workgroup where there are under two workgroups a CU ([16, 2048] x [8192, 2048], two a CU: 9.7 us with 8
+// waves, 11.7 with 16)
+template <bool F16, int MT>
+int launch_skinny_rows(hipStream_t st, const GemmShape &s, int64_t z, const void *a, const void *b, void *out, int dtype) {
+    if ((s.n + 15) / 16 * z >= 512) return launch_skinny_waves<F16, MT, 8>(st, s, z, a, b, out, dtype);
+    return launch_skinny_waves<F16, MT, 16>(st, s, z, a, b, out, dtype);
+}
+
+template <bool F16>
+int launch_skinny(hipStream_t st, const GemmShape &s, int64_t z, const void *a, const void *b, void *out, int dtype) {
+    if (s.m <= 16) return launch_skinny_rows<F16, 1>(st, s, z, a, b, out, dtype);
+    if (s.m <= 32) return launch_skinny_rows<F16, 2>(st, s, z, a, b, out, dtype);
+    return launch_skinny_rows<F16, 4>(st, s, z, a, b, out, dtype);
+}
+
 template <bool F16, bool AT, bool BT>
 int launch_mfma_layout(hipStream_t st, int cfg, GemmShape s, int64_t z, const void *a, const void *b, void *out, int dtype) {
     switch (cfg) {
@@ -382,6 +423,11 @@ int gemm_on(hipStream_t st, const nhip_gemm_desc *d, const void *a, const void *
              d->k % 64) ||
             ((cfg == kStream8w32 || cfg == kStream8wX || cfg == kStream8wP || cfg == kStream4wX) && d->k % 32))
             return fail("nhip_gemm: the streamed configs need k to be a multiple of their k tile");
+        if (cfg == kSkinny) {
+            if (!skinny_ok(d) || at || bt) return fail("nhip_gemm: config 16 takes at most 64 rows, both operands contiguous along k");
+            return d->a_dtype == NHIP_F16 ? launch_skinny<true>(st, s, z, a, b, out, d->d_dtype)
+                                          : launch_skinny<false>(st, s, z, a, b, out, d->d_dtype);
+        }
         if (d->a_dtype == NHIP_F16) return launch_mfma<true>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
         return launch_mfma<false>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
     }

@@ -249,3 +249,30 @@ def test_float32_fold_is_bit_exact_in_every_layout(hip, at, bt, m, n, k, z, out)
             bits = D.bf16_bits(want) if out == nv.NHIP_BF16 else want.astype(np.float16).view(np.uint16)
         ok = ~np.isnan(want)
         assert np.array_equal(got[ok], bits[ok]) and ok.sum() >= (m - 1) * n
+
+
+@pytest.mark.parametrize("m,n,k,z,out,dt", [
+    (1, 1, 8, 1, nv.NHIP_F32, nv.NHIP_BF16), (1, 17, 64, 1, nv.NHIP_F32, nv.NHIP_F16), (3, 8200, 512, 1, nv.NHIP_F32, nv.NHIP_BF16),
+    (16, 100, 1032, 2, nv.NHIP_BF16, nv.NHIP_BF16), (17, 640, 2120, 1, nv.NHIP_F32, nv.NHIP_F16),
+    (32, 48, 8200, 1, nv.NHIP_F32, nv.NHIP_BF16), (33, 130, 72, 1, nv.NHIP_F16, nv.NHIP_F16), (64, 1000, 2040, 1, nv.NHIP_F32, nv.NHIP_BF16)])
+def test_few_rows(hip, m, n, k, z, out, dt):
+    """Dots of up to 64 rows by default and as config 16: one, two and four 16-row groups, 8 and 16 waves a workgroup,
+    ragged columns, k of under one and many 64-element chunks with remainders, batches, output types; against
+    float64."""
+    rng = np.random.default_rng(m + n + k)
+    bits = D.bf16_bits if dt == nv.NHIP_BF16 else lambda x: x.astype(np.float16).view(np.uint16)
+    wide = D.bf16_to_f32 if dt == nv.NHIP_BF16 else lambda x: x.view(np.float16).astype(np.float32)
+    a, b = (bits(rng.standard_normal(s).astype(np.float32)) for s in ((z, m, k), (z, n, k)))
+    want = np.matmul(wide(a).astype(np.float64), wide(b).astype(np.float64).transpose(0, 2, 1))
+    scale = np.matmul(np.abs(wide(a)).astype(np.float64), np.abs(wide(b)).astype(np.float64).transpose(0, 2, 1))
+    for cfg in (-1, 16):
+        da, db, dd = Dev(a), Dev(b), Dev(nbytes=z * m * n * 4)
+        desc = _desc(m, n, k, k, 1, 1, k, dt=dt, out=out, cfg=cfg, batch=(z,), sa=(m * k,), sb=(n * k,), sd=(m * n,))
+        nv.call("nhip_gemm", C.byref(desc), da.ptr, db.ptr, dd.ptr)
+        if out == nv.NHIP_F32:
+            assert np.all(np.abs(dd.get((z, m, n), np.float32) - want) <= k * 2.0**-24 * scale)
+        else:
+            raw = dd.get((z, m, n), np.uint16)
+            got = D.bf16_to_f32(raw) if out == nv.NHIP_BF16 else raw.view(np.float16).astype(np.float32)
+            ulp = 2.0**-8 if out == nv.NHIP_BF16 else 2.0**-11
+            assert np.all(np.abs(got - want) <= ulp * np.abs(want) + k * 2.0**-24 * scale + 1e-6)
