@@ -1834,3 +1834,80 @@ class GemmEpilogueKernel:
             "}",
         ]
         return "\n".join(lines)
+
+
+class SmallGemmEpilogueKernel:
+    """A float32 fold (``gemm_fold_tile``) or a dot of few rows (``gemm_skinny_tile``) whose store is a fused loop step,
+    an element at a time: the loop's body runs on the dot's sum rounded to the dot's output dtype and writes the
+    loop's outputs (plus the dot's own result when anything else reads it). ``kind`` is ``("fold", rows a wave, A along
+    k, B along n)`` or ``("skinny", f16, 16-row groups, waves)``: the launch nhip_gemm would make."""
+
+    def __init__(self, graph, dot_step, loop_step, desc, kind, store_dot, views, out_views, aliased=frozenset()):
+        self.graph, self.dot, self.loop, self.desc, self.kind = graph, dot_step, loop_step, desc, kind
+        self.store_dot, self.views, self.out_views, self.aliased = store_dot, views, out_views, aliased
+        self.far = frozenset()  # as LoopKernel.far
+        self.name = "KNAME"
+        if kind[0] == "fold":
+            self.tiles = (-(-desc.m // (4 * kind[1])), -(-desc.n // 64))
+            self.grid, self.block = (self.tiles[0] * self.tiles[1], 1, 1), (256, 1, 1)
+        else:
+            self.tiles = (1, -(-desc.n // 16))
+            self.grid, self.block = (self.tiles[1], 1, 1), (64 * kind[3], 1, 1)
+        self.lds = 0
+        self.args = []
+
+    def source(self):
+        g, loop, d = self.graph, self.loop, self.desc
+        dv = self.dot.nodes[0].output
+        ddt = g.types[dv].dtype
+        lin = [v for v in loop.inputs if v != dv]
+        lk = LoopKernel(g, loop, "KNAME", {v: self.views[v] for v in lin}, self.out_views, self.aliased)
+        em = Emitter(g, loop.nodes, {v: (k, self.views[v]) for k, v in enumerate(lin)})
+        em.outputs = set(loop.outputs)
+        em.vec = 1
+        dname = em.tmp("d")
+        em.emit(f"const float {dname} = {em.round('acc', ddt) if ddt != 'float32' else 'acc'};")
+
+        def given(idx):
+            if idx[0] == "rc" and idx[1] == "r" and idx[2] == "c":
+                return dname
+            raise Unfusable(dv, "the fused loop reads the dot's result at another index")
+
+        em.given[dv] = given
+        em.rows, em.rows_uniform = (d.m, d.n), False
+        values = [em.value(v, ("rc", "r", "c", "c", 0)) for v in loop.outputs]
+        outs = ([dv] if self.store_dot else []) + list(loop.outputs)
+        values = ([dname] if self.store_dot else []) + values
+        stores = [f"out{k}[{lk._out_addr(self.out_views[v], g.types[v].shape, 'base')}] = {_store(x, g.types[v].dtype)};"
+                  for k, (v, x) in enumerate(zip(outs, values))]
+        self.args = [("in", u) for u in self.dot.nodes[0].inputs[:2]] + [("in", v) for v in lin] + [("out", v) for v in outs]
+        fields = [f"const {STORE_T[g.types[v].dtype]}*{_restrict(v, self.aliased)} in{k}" for k, v in enumerate(lin)]
+        fields += [f"{STORE_T[g.types[v].dtype]}*{_restrict(v, self.aliased)} out{k}" for k, v in enumerate(outs)]
+        init = ", ".join([f"in{k}" for k in range(len(lin))] + [f"out{k}" for k in range(len(outs))])
+        flag = {True: "true", False: "false"}
+        if self.kind[0] == "fold":
+            _, rows, ak, bn = self.kind
+            operand, call = "float", f"gemm_fold_tile<{rows}, {flag[ak]}, {flag[bn]}>"
+        else:
+            _, f16, groups, waves = self.kind
+            operand, call = "uint16_t", f"gemm_skinny_tile<{flag[f16]}, {groups}, {waves}>"
+        params = [f"const {operand}* __restrict__ a", f"const {operand}* __restrict__ b"] + fields
+        lines = [
+            f'#include "gemm_{self.kind[0]}.h"',
+            "struct EpiKNAME {",
+            *[f"  {f};" for f in fields],
+            "  template <class F> __device__ __forceinline__ void visit(F &&f) const { f(*this); }",
+            "  __device__ __forceinline__ void operator()(const nhipk::GemmShape &, int64_t, int64_t r, int64_t c, float acc) const {",
+            f"    const int64_t base = r * {d.n}LL + c;",
+            *["    " + l for l in lk._vec_prologue(em, 1, lin) + em.lines + stores],
+            "  }",
+            "};",
+            f'extern "C" __global__ __launch_bounds__({self.block[0]}) void KNAME({", ".join(params)}) {{',
+            "  nhipk::GemmShape s;",
+            f"  s.m = {d.m}LL; s.n = {d.n}LL; s.k = {d.k}LL; s.nbatch = 0; s.a_m = {d.a_m}LL; s.a_k = {d.a_k}LL; "
+            f"s.b_k = {d.b_k}LL; s.b_n = {d.b_n}LL; s.d_m = {d.n}LL; s.d_n = 1; s.tiles_m = {self.tiles[0]}; "
+            f"s.tiles_n = {self.tiles[1]}; s.d_split = 0;",
+            f"  nhipk::{call}(s, a, b, EpiKNAME{{{init}}});",
+            "}",
+        ]
+        return "\n".join(lines)

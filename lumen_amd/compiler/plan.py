@@ -64,6 +64,31 @@ def _skinny(d) -> bool:
     return d.m <= 64 and d.a_k == 1 and d.b_k == 1 and groups * d.n <= 24576 and (groups <= 2 or d.k <= 2048)
 
 
+# float32 dots up to this many multiply-adds (15 us on the chip) take their consumer into the store: a launch and a
+# pass over the result are a tenth of such a call or more ([256, 512] x [512, 1024] with its relu: 15.5 -> 11.6 us)
+SMALL_FOLD_MACS = 1 << 27
+
+
+def _small_kind(d, ops):
+    """The SmallGemmEpilogueKernel ``kind`` nhip_gemm runs an unbatched dot as (kernels.hip: gemm_on's choice of
+    gemm_fold and its fold_rows, gemm_skinny's waves), or None where it takes another kernel."""
+    if not 0 < d.k < 1 << 30 or d.a_dtype != d.b_dtype:
+        return None
+    if d.a_dtype == NHIP_DT["float32"]:
+        if d.m * d.n * d.k > SMALL_FOLD_MACS:
+            return None
+        if (d.a_k != 1 and d.a_m != 1) or (d.b_k != 1 and d.b_n != 1):
+            return None
+        ak, rm = d.a_k == 1, 4 if d.a_k == 1 else 8
+        while rm > 1 and (d.m < rm or -(-d.m // rm) * -(-d.n // 64) < (2048 if ak else 1024)):
+            rm //= 2
+        return "fold", rm, ak, d.b_n == 1
+    if not _mfma_layout(d) or not _skinny(d) or any((loc.offset * D.size_of(loc.dtype)) % 16 for loc in ops[:2]):
+        return None
+    return "skinny", d.a_dtype == NHIP_DT["float16"], 1 if d.m <= 16 else 2 if d.m <= 32 else 4, \
+        8 if -(-d.n // 16) >= 512 else 16
+
+
 def _contig(shape):
     return codegen._contig(shape)
 
@@ -495,7 +520,8 @@ class Plan:
 
     def _epilogue_layout(self, st):
         """``(desc, at, bt, f16)`` when dot step ``st`` can run as a streamed GEMM with a generated epilogue
-        (2-D bf16/f16 operands, k a multiple of 64, one k split, operand rows 16-byte aligned), else None."""
+        (2-D bf16/f16 operands, k a multiple of 64, one k split, operand rows 16-byte aligned), ``(desc, kind)`` when
+        it runs as a SmallGemmEpilogueKernel, else None."""
         from lumen_amd import native as nv
 
         n = st.nodes[0]
@@ -508,6 +534,9 @@ class Plan:
             d, ops = self._gemm_desc(n)
         except NotImplementedError:
             return None
+        small = _small_kind(d, ops)
+        if small is not None:
+            return d, small
         if d.a_dtype != d.b_dtype or d.a_dtype not in (nv.NHIP_BF16, nv.NHIP_F16) or d.k % 64 or d.n % 4:
             return None
         if -(-d.m // 256) * -(-d.n // 256) < self.EPI_MIN_TILES:
@@ -587,7 +616,8 @@ class Plan:
                 readers.setdefault(u, []).append(st)
         gone = set()
         for st in self.steps:
-            if st.kind != "dot" or getattr(st, "epi", None) is None or getattr(st, "epi_colsum", None):
+            if st.kind != "dot" or getattr(st, "epi", None) is None or getattr(st, "epi_colsum", None) \
+                    or len(st.epi_layout) == 2:
                 continue
             shape = g.types[st.nodes[0].output].shape
             for u in st.epi.outputs:
@@ -689,11 +719,20 @@ class Plan:
                 self.sources[si] = codegen.HEADER + body.replace("KNAME", name)
                 continue
             if st.kind == "dot" and getattr(st, "epi", None) is not None:
-                d, at, bt, f16 = st.epi_layout
-                d, _ = self._gemm_desc(st.nodes[0])
                 lin = [v for v in st.epi.inputs if v != st.nodes[0].output]
                 views = {v: self.loc[v].view() for v in lin}
                 outs = {v: self.loc[v].view() for v in st.outputs}
+                if len(st.epi_layout) == 2:
+                    d, _ = self._gemm_desc(st.nodes[0])
+                    k = codegen.SmallGemmEpilogueKernel(g, st, st.epi, d, st.epi_layout[1], st.store_dot, views, outs,
+                                                        aliased=self.aliased)
+                    body = k.source()
+                    k.name = st.name = f"gemm_{st.epi_layout[1][0]}_{hashlib.sha1(body.encode()).hexdigest()[:10]}"
+                    self.kernels[si] = k
+                    self.sources[si] = codegen.HEADER + body.replace("KNAME", k.name)
+                    continue
+                d, at, bt, f16 = st.epi_layout
+                d, _ = self._gemm_desc(st.nodes[0])
                 k = codegen.GemmEpilogueKernel(g, st, st.epi, d, at, bt, f16, st.store_dot, views, outs,
                                                colsum=getattr(st, "epi_colsum", None), aliased=self.aliased)
                 k.far = far

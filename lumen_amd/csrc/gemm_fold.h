@@ -37,10 +37,10 @@ struct ScalarVec<1> {
 };
 
 // AK: A contiguous along k, else along m. BN: B contiguous along n, else along k.
-// Needs m >= RM and k < 2^30.
+// Needs m >= RM and k < 2^30. `epi.visit(f)` calls f with the store: st(s, batch offset, row, column, sum).
 template <int RM, bool AK, bool BN, class Epi>
-__global__ __launch_bounds__(256) void gemm_fold(GemmShape s, const float *__restrict__ a, const float *__restrict__ b,
-                                                 Epi epi) {
+__device__ __forceinline__ void gemm_fold_tile(const GemmShape &s, const float *__restrict__ a, const float *__restrict__ b,
+                                               const Epi &epi) {
     constexpr int KB = 32;                           // k of a staged B tile
     constexpr int KC = RM <= 2 ? 16 : 32 / RM;       // k of a register chunk: 2 RM KC <= 64 SGPRs
     constexpr int CH = KB / KC;
@@ -52,8 +52,9 @@ __global__ __launch_bounds__(256) void gemm_fold(GemmShape s, const float *__res
     tile_of(blockIdx.x, s.tiles_m, s.tiles_n, tm, tn);
     int64_t oa, ob, od;
     batch_offsets(s, blockIdx.y, oa, ob, od);
-    // the wave's rows: the last RM ones where fewer are left (rows computed twice are stored twice, alike)
-    const int64_t m0 = min(int64_t(tm) * (4 * RM) + wave * RM, s.m - RM), n0 = int64_t(tn) * 64;
+    // the wave's rows: the last RM ones where fewer are left, of which those before `own` are another wave's to store
+    const int64_t own = int64_t(tm) * (4 * RM) + wave * RM;
+    const int64_t m0 = min(own, s.m - RM), n0 = int64_t(tn) * 64;
     const int ktot = int(s.k);
 
     // B's tile at k0, 16 bytes at a time along its contiguous axis: thread t takes 4 columns of rows t / 16 and 16
@@ -187,8 +188,15 @@ __global__ __launch_bounds__(256) void gemm_fold(GemmShape s, const float *__res
     if (col >= s.n) return;
     epi.visit([&](auto out) {
 #pragma unroll
-        for (int r = 0; r < RM; ++r) out(s, od, m0 + r, col, acc[r]);
+        for (int r = 0; r < RM; ++r)
+            if (m0 + r >= own) out(s, od, m0 + r, col, acc[r]);
     });
+}
+
+template <int RM, bool AK, bool BN, class Epi>
+__global__ __launch_bounds__(256) void gemm_fold(GemmShape s, const float *__restrict__ a, const float *__restrict__ b,
+                                                 Epi epi) {
+    gemm_fold_tile<RM, AK, BN>(s, a, b, epi);
 }
 
 }  // namespace nhipk

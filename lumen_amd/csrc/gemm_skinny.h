@@ -23,10 +23,11 @@ __device__ __forceinline__ f32x4_t mfma16(uint4 a, uint4 b, f32x4_t c) {
                                                         0, 0, 0);
 }
 
-// MT: 16-row groups of A (m <= 16 MT). Needs k % 8 == 0 and 16-byte aligned rows.
-template <bool F16, int MT, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_skinny(GemmShape s, const uint16_t *__restrict__ a,
-                                                        const uint16_t *__restrict__ b, AnyStore out) {
+// MT: 16-row groups of A (m <= 16 MT). Needs k % 8 == 0 and 16-byte aligned rows. `epi.visit(f)` calls f with the
+// store: st(s, batch offset, row, column, sum).
+template <bool F16, int MT, int NW, class Epi>
+__device__ __forceinline__ void gemm_skinny_tile(const GemmShape &s, const uint16_t *__restrict__ a,
+                                                 const uint16_t *__restrict__ b, const Epi &epi) {
     constexpr int U = MT >= 4 ? 2 : 4;  // chunks of 64 k in flight
     __shared__ f32x4_t sums[NW][MT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
@@ -84,11 +85,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny(GemmShape s, const uint16
     for (int w = 1; w < NW; ++w) v += sums[w][wave][lane];
     const int64_t col = n0 + l16, row = 16 * wave + 4 * g;
     if (col >= s.n) return;
-    out.visit([&](auto st) {
+    epi.visit([&](auto st) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (row + e < s.m) st(s, od, row + e, col, v[e]);
     });
+}
+
+template <bool F16, int MT, int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_skinny(GemmShape s, const uint16_t *__restrict__ a,
+                                                        const uint16_t *__restrict__ b, AnyStore out) {
+    gemm_skinny_tile<F16, MT, NW>(s, a, b, out);
 }
 
 }  // namespace nhipk

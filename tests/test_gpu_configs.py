@@ -588,3 +588,49 @@ def test_norm_backward_row_kernel_sums_its_weight_gradient(hip, rows, cols):
     assert np.abs(dx - want).max() <= 1e-5 * np.abs(want).max()
     bound = (rows + 8) * 2.0**-24 * np.abs(terms).sum(0)
     assert np.all(np.abs(dw - terms.sum(0)) <= bound)
+
+
+@pytest.mark.parametrize("m,k,n,dt", [(1, 33, 5, "float32"), (3, 64, 70, "float32"), (250, 97, 129, "float32"),
+                                      (1030, 40, 100, "float32"), (1, 64, 40, "bfloat16"), (16, 520, 300, "float16"),
+                                      (33, 128, 1000, "bfloat16"), (64, 72, 24, "bfloat16")])
+def test_small_dots_take_their_consumer_into_the_store(hip, m, k, n, dt):
+    """float32 folds and dots of few rows with an elementwise consumer that reads a row and a column operand, the
+    result itself returned too: one kernel, equal bit for bit to the two kernels it replaces."""
+    rng = np.random.default_rng(m + n + k)
+    x, w = (L.tensor(rng.standard_normal(s).astype(np.float32), dt) for s in ((m, k), (n, k)))
+    b, r = (L.tensor(rng.standard_normal(s).astype(np.float32), "float32") for s in ((n,), (m, 1)))
+
+    def fn(x, w, b, r):
+        y = F.matmul(x, w.t(), "float32", "float32")
+        return F.gelu(y + b) * r, y
+
+    args = [t.to(device="hip") for t in (x, w, b, r)]
+    outs = []
+    for fuse in (True, False):
+        with L.config.compiler.patch(epilogue_fusion=fuse):
+            f = L.compile(fn, device="hip")
+            outs.append([L.to_numpy(t) for t in f(*args)])
+            dots = [st for st in f.plan.steps if st.kind == "dot"]
+            assert (getattr(dots[0], "epi", None) is not None) == fuse
+    for a, c in zip(*outs):
+        np.testing.assert_array_equal(a, c)
+
+
+def test_small_update_in_place_reads_each_weight_once(hip):
+    """w - lr x^T y written over w by the fold's store: rows that two waves compute (m not a multiple of the rows a
+    wave) are stored by one of them only."""
+    from lumen_amd.compiler.plan import Plan
+    rng = np.random.default_rng(3)
+    for m, k, n in ((5, 40, 300), (1027, 16, 200)):
+        w, x, y = (rng.standard_normal(s).astype(np.float32) for s in ((m, n), (m, k), (k, n)))
+        g = L.make_graph(lambda w, x, y: (w - 0.5 * F.matmul(x, y, "float32", "float32"),))(
+            *[L.from_numpy(a) for a in (w, x, y)])
+        plan = Plan(g, "hip:0", donate={0: 0})
+        assert plan.in_place_outputs == {0: 0} and [st.kind for st in plan.steps] == ["dot"]
+        dev = [L.from_numpy(a).to("hip") for a in (w, x, y)]
+        ws = L.empty([max(1, plan.workspace_bytes)], "uint8", "hip")
+        plan.run_in(ws.data_ptr(), [t.data_ptr() for t in dev])
+        fold = np.zeros((m, n), np.float32)
+        for i in range(k):
+            fold += x[:, i, None] * y[i]
+        np.testing.assert_allclose(L.to_numpy(dev[0]), w - np.float32(0.5) * fold, rtol=0, atol=1e-6)
