@@ -188,7 +188,23 @@ struct FragLayout {
     static constexpr int pitch = P;
 };
 
-template <bool F16, int BM, int BN, int BK, int WM, int WN, bool AT, bool BT, class Epi>
+// 8 elements at `p`, of which `n` (any number, at least 1) are the operand's and the rest zeros: rows of any length
+// start at any 2-byte address, and their last chunk ends inside its 16 bytes.
+__device__ __forceinline__ uint4 load8_any(const uint16_t *p, int64_t n) {
+    typedef uint32_t any4 __attribute__((ext_vector_type(4), aligned(2)));
+    if (n >= 8) {
+        const any4 v = *reinterpret_cast<const any4 *>(p);
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 7; ++i)
+        if (i < n) w[i / 2] |= uint32_t(p[i]) << (16 * (i & 1));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// ANY: operands of any row length and alignment (load8_any), else 16-byte aligned rows of a multiple of 8 elements.
+template <bool F16, int BM, int BN, int BK, int WM, int WN, bool AT, bool BT, class Epi, bool ANY = false>
 __global__ __launch_bounds__(WM *WN * 64) void gemm_mfma(GemmShape s, const uint16_t *__restrict__ a,
                                                            const uint16_t *__restrict__ b, Epi epi) {
     constexpr int T = WM * WN * 64;
@@ -224,7 +240,8 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_mfma(GemmShape s, const uint
             else gm = m0 + line, gk = k0 + ch * 8;
             bool ok = gm < s.m && gk < s.k;
             const uint16_t *src = AT ? pa + gk * s.a_k + gm : pa + gm * s.a_m + gk;
-            ra[v] = ok ? *reinterpret_cast<const uint4 *>(src) : make_uint4(0, 0, 0, 0);
+            if constexpr (ANY) ra[v] = ok ? load8_any(src, AT ? s.m - gm : s.k - gk) : make_uint4(0, 0, 0, 0);
+            else ra[v] = ok ? *reinterpret_cast<const uint4 *>(src) : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int v = 0; v < VB; ++v) {
@@ -234,7 +251,8 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_mfma(GemmShape s, const uint
             else gn = n0 + line, gk = k0 + ch * 8;
             bool ok = gn < s.n && gk < s.k;
             const uint16_t *src = BT ? pb + gk * s.b_k + gn : pb + gn * s.b_n + gk;
-            rb[v] = ok ? *reinterpret_cast<const uint4 *>(src) : make_uint4(0, 0, 0, 0);
+            if constexpr (ANY) rb[v] = ok ? load8_any(src, BT ? s.n - gn : s.k - gk) : make_uint4(0, 0, 0, 0);
+            else rb[v] = ok ? *reinterpret_cast<const uint4 *>(src) : make_uint4(0, 0, 0, 0);
         }
     };
     auto store = [&](int buf) {

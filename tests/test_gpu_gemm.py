@@ -276,3 +276,32 @@ def test_few_rows(hip, m, n, k, z, out, dt):
             got = D.bf16_to_f32(raw) if out == nv.NHIP_BF16 else raw.view(np.float16).astype(np.float32)
             ulp = 2.0**-8 if out == nv.NHIP_BF16 else 2.0**-11
             assert np.all(np.abs(got - want) <= ulp * np.abs(want) + k * 2.0**-24 * scale + 1e-6)
+
+
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k,z,dt,shift", [
+    (1, 1, 1, 1, nv.NHIP_BF16, 0), (3, 7, 5, 2, nv.NHIP_F16, 0), (65, 130, 67, 1, nv.NHIP_BF16, 1), (200, 75, 129, 3, nv.NHIP_F16, 1),
+    (2100, 2051, 61, 1, nv.NHIP_BF16, 0), (4097, 4099, 17, 1, nv.NHIP_BF16, 3), (64, 64, 64, 1, nv.NHIP_BF16, 1)])
+def test_16bit_operands_of_any_length_and_alignment(hip, at, bt, m, n, k, z, dt, shift):
+    """Row lengths that are no multiple of 8, operands that start off 16 bytes (``shift`` elements in), all three tile
+    sizes, every memory order, batches: against float64. The operands are followed by NaN bits, which no result
+    may take up."""
+    rng = np.random.default_rng(m + n + k)
+    bits = D.bf16_bits if dt == nv.NHIP_BF16 else lambda x: x.astype(np.float16).view(np.uint16)
+    wide = D.bf16_to_f32 if dt == nv.NHIP_BF16 else lambda x: x.view(np.float16).astype(np.float32)
+    a, b = (bits(rng.standard_normal(s).astype(np.float32)) for s in ((z, m, k), (z, k, n)))
+
+    def stored(x):
+        pad = np.full(shift + x.size + 64, 0x7FFF, np.uint16)
+        pad[shift:shift + x.size] = x.reshape(-1)
+        return Dev(pad)
+
+    da = stored(np.ascontiguousarray(a.transpose(0, 2, 1)) if at else a)
+    db = stored(b if bt else np.ascontiguousarray(b.transpose(0, 2, 1)))
+    dd = Dev(nbytes=z * m * n * 4)
+    desc = _desc(m, n, k, 1 if at else k, m if at else 1, n if bt else 1, 1 if bt else k, dt=dt, batch=(z,), sa=(m * k,),
+                 sb=(k * n,), sd=(m * n,))
+    nv.call("nhip_gemm", C.byref(desc), da.ptr + 2 * shift, db.ptr + 2 * shift, dd.ptr)
+    fa, fb = wide(a).astype(np.float64), wide(b).astype(np.float64)
+    scale = np.matmul(np.abs(fa), np.abs(fb))
+    assert np.all(np.abs(dd.get((z, m, n), np.float32) - np.matmul(fa, fb)) <= k * 2.0**-24 * scale)
