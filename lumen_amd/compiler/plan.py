@@ -484,9 +484,14 @@ class Plan:
                 st.splits, split_cfg = (1, None) if getattr(st, "epi", None) is not None else self._split_count(st.nodes[0])
                 if split_cfg is not None:
                     st.config = split_cfg
-                if st.splits > 1:
+                st.split_choices, st.scratch = [st.splits], 0
+                if st.splits > 1 or split_cfg is not None:
                     d, _ = self._gemm_desc(st.nodes[0])
-                    st.scratch = st.splits * max(1, math.prod(d.batch[i] for i in range(d.nbatch))) * d.m * d.n * 4
+                    if config.compiler.autotune and not config.compiler.memory_limit:
+                        st.split_choices = self._split_choices(d, st.splits)
+                most = max(st.split_choices + [st.splits])
+                if most > 1:
+                    st.scratch = most * max(1, math.prod(d.batch[i] for i in range(d.nbatch))) * d.m * d.n * 4
             if st.kind == "linear_cross_entropy":
                 st.scratch = self._lce_scratch(self._lce_desc(st.nodes[0]))
             if st.scratch:
@@ -1139,8 +1144,10 @@ class Plan:
         nv.call("nhip_gemm_config_count", C.byref(n_cfg))
         ev0, ev1 = nv.Event(), nv.Event()
         for st in self.steps:
-            if st.kind != "dot" or getattr(st, "splits", 1) > 1 or getattr(st, "epi", None) is not None \
-                    or getattr(st, "forced", False):
+            if st.kind != "dot" or getattr(st, "epi", None) is not None or getattr(st, "forced", False):
+                continue
+            choices = getattr(st, "split_choices", [1])
+            if len(choices) == 1 and getattr(st, "splits", 1) > 1:
                 continue
             try:
                 d, ops = self._gemm_desc(st.nodes[0])
@@ -1150,30 +1157,33 @@ class Plan:
             if d.a_dtype == nv.NHIP_F32 or d.m * d.n * d.k * z < self.AUTOTUNE_MACS:
                 continue
             key = (d.m, d.n, d.k, tuple(d.batch[i] for i in range(d.nbatch)), d.a_dtype, d.d_dtype,
-                   d.a_m == 1, d.a_k == 1, d.b_k == 1, d.b_n == 1, d.d_n == 1)
+                   d.a_m == 1, d.a_k == 1, d.b_k == 1, d.b_n == 1, d.d_n == 1, tuple(choices))
             if key not in Plan._tuned:
                 ptrs = []
                 for loc in ops:
                     base = workspace_ptr if loc.base[0] == "ws" else input_ptrs[loc.base[1]]
                     ptrs.append(base + loc.offset * D.size_of(loc.dtype))
-                best, best_ms = -1, float("inf")
-                for cfg in range(n_cfg.value):
-                    d.config = cfg
-                    try:
-                        nv.call("nhip_gemm", C.byref(d), *ptrs)  # warm-up; rejects configs the shape can't take
-                    except RuntimeError:
-                        continue
-                    ev0.record()
-                    for _ in range(3):
-                        nv.call("nhip_gemm", C.byref(d), *ptrs)
-                    ev1.record()
-                    ms = ev0.elapsed_ms(ev1) / 3
-                    # a later config must win by more than timing noise (3%), so near-ties pick the same
-                    # kernel run after run
-                    if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
-                        best, best_ms = cfg, ms
+                scratch = self.scratch.get(id(st))
+                ptrs.append(workspace_ptr + scratch.offset * 4 if scratch is not None else None)
+                best, best_ms = (-1, 1), float("inf")
+                for splits in choices:
+                    for cfg in range(n_cfg.value) if splits == 1 else (self.STREAM128, self.STREAM8W):
+                        d.config, d.splits = cfg, splits
+                        try:  # warm-up; rejects configs the shape can't take
+                            nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
+                        except RuntimeError:
+                            continue
+                        ev0.record()
+                        for _ in range(3):
+                            nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
+                        ev1.record()
+                        ms = ev0.elapsed_ms(ev1) / 3
+                        # a later config must win by more than timing noise (3%), so near-ties pick the same
+                        # kernel run after run
+                        if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
+                            best, best_ms = (cfg, splits), ms
                 Plan._tuned[key] = best
-            st.config = Plan._tuned[key]
+            st.config, st.splits = Plan._tuned[key]
 
     # Split-k policy: a bf16/f16 dot whose 256 x 256 output tiles cannot fill the 256 CUs is cut along k (in
     # powers of two, each part at least 1024 deep) until they do; its float32 partials live in the step's
@@ -1181,6 +1191,23 @@ class Plan:
     SPLIT_MIN_K = 1024
     SPLIT_MAX = 8
     STREAM128 = 9  # kernels.hip's kStream128
+    STREAM8W = 7  # kernels.hip's kStream8w
+    SPLIT_TUNED_MIN_K = 512
+    SPLIT_TUNED_BYTES = 256 << 20
+
+    def _split_choices(self, d, splits):
+        """The split counts the autotuner times for a dot the policy gives ``splits``: powers of two to SPLIT_MAX with
+        parts of at least SPLIT_TUNED_MIN_K and float32 partials within SPLIT_TUNED_BYTES. The policy only fills
+        the chip; whether that pays for writing and reading the partials depends on the shape: [8192, 2048] x [2048,
+        512] takes 28 us whole and 36 in two parts, [2048, 8192] x [8192, 512] 78 and 41 in eight."""
+        z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
+        if d.m * d.n * d.k * z < self.AUTOTUNE_MACS or -(-d.m // 256) * -(-d.n // 256) * z >= 256 or _skinny(d):
+            return [splits]
+        s = [1]
+        while s[-1] < self.SPLIT_MAX and d.k % (128 * s[-1]) == 0 and d.k // (2 * s[-1]) >= self.SPLIT_TUNED_MIN_K \
+                and 8 * s[-1] * z * d.m * d.n <= self.SPLIT_TUNED_BYTES:
+            s.append(2 * s[-1])
+        return s
 
     def _split_count(self, n):
         lhs, rhs, out = self.loc[n.inputs[0]], self.loc[n.inputs[1]], self.loc[n.output]
@@ -1204,7 +1231,7 @@ class Plan:
         while (tiles * s * 2 <= 512 and s < self.SPLIT_MAX and d.k % (64 * s * 2) == 0
                and d.k // (s * 2) >= self.SPLIT_MIN_K):
             s *= 2
-        return s, (self.STREAM128 if s > 1 else None)
+        return s, (self.STREAM128 if s > 1 else -1)
 
     def run_in(self, workspace_ptr: int, input_ptrs: list):
         """Queues the plan on the stream: inputs are device pointers in graph-input order. The first run

@@ -576,3 +576,20 @@ def test_norm_weight_gradient_sums_join_the_row_kernel():
     ids = L.empty([W.TINY.batch, W.TINY.seq], "int64", "meta")
     p = Plan(trace(W.train_step, (model, opt, ids, ids)).graph, build_kernels=False)
     assert sum(len(st.colsums) for st in p.steps) >= 2
+
+
+def test_split_counts_are_timed_where_the_dot_is_large():
+    """A large dot whose 256 x 256 tiles do not fill the chip has scratch for every split count the autotuner times; a
+    small one, one that fills it, and a plan with a memory limit keep the policy's count."""
+    def dot(m, n, k):
+        p = _plan(lambda x, w: F.matmul(x, w.t(), "float32", "bfloat16"), ((m, k), "bfloat16"), ((n, k), "bfloat16"))
+        return next(st for st in p.steps if st.kind == "dot")
+
+    st = dot(8192, 512, 2048)
+    assert st.split_choices == [1, 2, 4] and st.scratch == 4 * 8192 * 512 * 4
+    assert dot(512, 2048, 8192).split_choices == [1, 2, 4, 8]
+    assert dot(8192, 8192, 512).split_choices == [1] and dot(8192, 8192, 512).scratch == 0
+    assert dot(256, 512, 1024).split_choices == [1] and dot(1000, 512, 8000).split_choices[0] == 1
+    with L.config.compiler.patch(memory_limit=1 << 40):
+        st = dot(512, 2048, 8192)
+        assert st.split_choices == [st.splits] == [8]
