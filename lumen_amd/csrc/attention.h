@@ -125,6 +125,13 @@ __device__ __forceinline__ int kv_off(int r, int col) {
     return r * (D * 2) + ((((col >> 3) ^ kv_swz<D>(r))) << 4) + ((col & 7) << 1);
 }
 
+// The larger of a lane's and its other half-wave's value (lane ^ 32), by a register swap instead of a trip through LDS.
+__device__ __forceinline__ float max_halves(float x) {
+    typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+    const u32x2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 // Zeros `elems` 16-bit elements of LDS (a multiple of 8) when the kernel's tiles can be partial (rows past the
@@ -194,13 +201,16 @@ template <int NW, int D = 128> struct FwdOccupancy {
     static constexpr int kBlocks = D > 128 ? 1 : (NW >= 8 ? 1 : (NW >= 4 ? 2 : 4));
 };
 
-template <int D, bool F16, bool CAUSAL, int NW = 4>
-__global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash_fwd_kernel(AttnParams p) {
+// The two stages are arrays of their own, named by a constant in the loop below: were they halves of one array, every
+// LDS read would be taken to alias the loads just issued into the other half and wait for them (s_waitcnt vmcnt(0)
+// before the tile's first read), so that nothing overlapped.
+template <int D, bool F16, bool CAUSAL, int NW>
+__device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     constexpr int QB = 32 * NW;  // queries a workgroup
     constexpr int BN = 64;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int TILE = BN * D;  // elements
-    __shared__ __align__(1024) uint16_t smem[4 * TILE];  // K0 V0 K1 V1
+    __shared__ __align__(1024) uint16_t stage0[2 * TILE], stage1[2 * TILE];  // K, V
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
     const int g = lane >> 4, s16 = lane & 15;
@@ -228,10 +238,11 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
     if (CAUSAL) full_end = min(full_end, q0 + shift + 1);
     const int nfull = full_end > 0 ? int(full_end / BN) : 0;
 
-    zero_tiles(smem, 4 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
+    zero_tiles(stage0, 2 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
+    zero_tiles(stage1, 2 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
     if (ntiles > 0) {
-        load_tile_async<D, NW>(kp, p.k_s, 0, p.sk, smem, wave, lane, p.hd);
-        load_tile_async<D, NW>(vp, p.v_s, 0, p.sk, smem + TILE, wave, lane, p.hdv);
+        load_tile_async<D, NW>(kp, p.k_s, 0, p.sk, stage0, wave, lane, p.hd);
+        load_tile_async<D, NW>(vp, p.v_s, 0, p.sk, stage0 + TILE, wave, lane, p.hdv);
     }
 
     uint4 qf[DS];
@@ -248,18 +259,16 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
     const float c2 = p.scale * 1.4426950408889634f;  // scale * log2(e)
     float m = -1e30f, l = 0.0f;                       // running max (base 2, scaled) and sum
 
-    for (int kt = 0; kt < ntiles; ++kt) {
+    auto tile = [&](int kt, const uint16_t *Ks, uint16_t *nk) __attribute__((always_inline)) {
         const int64_t k0 = int64_t(kt) * BN;
-        const uint16_t *Ks = smem + (kt & 1) * 2 * TILE;
         const uint16_t *Vs = Ks + TILE;
         __builtin_amdgcn_s_waitcnt(0);  // this thread's loads of tile kt have landed
         __syncthreads();                // ... and every thread's; tile kt-1's buffer is free
         if (kt + 1 < ntiles) {
-            uint16_t *nk = smem + ((kt + 1) & 1) * 2 * TILE;
             load_tile_async<D, NW>(kp, p.k_s, k0 + BN, p.sk, nk, wave, lane, p.hd);
             load_tile_async<D, NW>(vp, p.v_s, k0 + BN, p.sk, nk + TILE, wave, lane, p.hdv);
         }
-        if (CAUSAL && k0 > wq_last + shift) continue;  // every key of the tile is masked for this wave
+        if (CAUSAL && k0 > wq_last + shift) return;  // every key of the tile is masked for this wave
         const char *Kb = reinterpret_cast<const char *>(Ks);
         const char *Vb = reinterpret_cast<const char *>(Vs);
 
@@ -276,7 +285,7 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
         }
         float mx = -INFINITY;
         if (kt >= nfull) {  // diagonal or ragged tile
-            const int64_t lim = min(CAUSAL ? qi + shift : p.sk - 1, p.sk - 1) - k0 - 4 * h;
+            const int lim = int(max(min(min(CAUSAL ? qi + shift : p.sk - 1, p.sk - 1) - k0 - 4 * h, int64_t(BN)), int64_t(-1)));
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -289,7 +298,7 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[ks][e]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
+        mx = max_halves(mx) * c2;
         // raise m only when some row's maximum outgrew it by 2^8
         if (__any(mx > m + 8.0f)) {
             const float mnew = fmaxf(m, mx);
@@ -301,7 +310,7 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
                 for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
             m = mnew;
         }
-        float rs = 0.0f;
+        float rs = 0.0f;  // this half-wave's keys: the halves' sums are added at the end
         uint4 pb[4];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
@@ -317,7 +326,7 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
                 }
                 pb[2 * ks + half] = make_uint4(w[0], w[1], w[2], w[3]);
             }
-        l += rs + __shfl_xor(rs, 32, 64);
+        l += rs;
 #pragma unroll
         for (int t2 = 0; t2 < 4; ++t2) {
             const int key = 16 * t2 + 4 * h + s16 / 4;
@@ -330,8 +339,13 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
                 acc[dt] = mfma32<F16>(make_uint4(xa.x, xa.y, ya.x, ya.y), pb[t2], acc[dt]);
             }
         }
+    };
+    for (int kt = 0; kt < ntiles; kt += 2) {
+        tile(kt, stage0, stage1);
+        if (kt + 1 < ntiles) tile(kt + 1, stage1, stage0);
     }
 
+    l += __shfl_xor(l, 32, 64);
     if (!qvalid) return;
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     uint16_t *op = p.o + b * p.o_b + n * p.o_n + qi * p.o_s;
@@ -345,6 +359,11 @@ __global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash
             *reinterpret_cast<uint2 *>(op + 32 * dt + 8 * e4 + 4 * h) = make_uint2(w0, w1);
         }
     if (h == 0 && p.lse) p.lse[(b * p.heads + n) * p.sq + qi] = l > 0.0f ? (m + __log2f(l)) * 0.6931471805599453f : -INFINITY;
+}
+
+template <int D, bool F16, bool CAUSAL, int NW = 4>
+__global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash_fwd_kernel(AttnParams p) {
+    flash_fwd_body<D, F16, CAUSAL, NW>(p);
 }
 
 template <bool F16>

@@ -105,16 +105,7 @@ static int launch_split_kernel(hipStream_t s, const nhipk::AttnParams &p, const 
         sp.splits = 1;
         sp.keytiles = (d->sk + 31) / 32;
     }
-    constexpr int lds = nhipk::flash_split_lds_bytes<D>();
-    auto kern = nhipk::flash_split_kernel<D, F16, CAUSAL>;
-    static bool attr = false;
-    if (!attr) {
-        if (check(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-                  "hipFuncSetAttribute"))
-            return 1;
-        attr = true;
-    }
-    hipLaunchKernelGGL(kern, dim3(unsigned(units * sp.splits)), dim3(256), lds, s, p, sp);
+    hipLaunchKernelGGL((nhipk::flash_split_kernel<D, F16, CAUSAL>), dim3(unsigned(units * sp.splits)), dim3(256), 0, s, p, sp);
     if (check(hipGetLastError(), "flash split launch")) return 1;
     if (sp.splits == 1) return 0;
     hipLaunchKernelGGL((nhipk::flash_combine_kernel<F16>), dim3(unsigned((d->batch * d->kv_heads * sp.rows + 3) / 4)),

@@ -70,14 +70,11 @@ __device__ __forceinline__ void load_pair32(const AttnParams &p, const uint16_t 
     load_tile32<D>(vp, p.v_s, k0, p.sk, dst + 32 * D, lane, p.hdv);
 }
 
-// LDS: four waves' rings of two (K, V) tile pairs; the same memory holds the waves' sums at the end.
-template <int D>
-constexpr int flash_split_lds_bytes() { return 4 * 2 * 2 * 32 * D * 2; }
-
+// As in flash_fwd_body the two stages are arrays of their own; the first holds the waves' sums at the end.
 template <int D, bool F16, bool CAUSAL>
-__global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitParams sp) {
+__device__ __forceinline__ void flash_split_body(const AttnParams &p, const SplitParams &sp) {
     constexpr int BN = 32, DS = D / 16, DT = D / 32, TILE = BN * D;
-    extern __shared__ __align__(1024) uint16_t split_lds[];
+    __shared__ __align__(1024) uint16_t rings0[4][2 * TILE], rings1[4][2 * TILE];
     __shared__ float2 ml[4][32];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, l32 = lane & 31, g = lane >> 4, s16 = lane & 15;
@@ -105,9 +102,12 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
     const int64_t t0 = split * sp.keytiles;
     const int64_t t1 = min(t0 + sp.keytiles, (kend + BN - 1) / BN);
 
-    uint16_t *ring = split_lds + wave * 4 * TILE;
+    uint16_t *const ring0 = rings0[wave], *const ring1 = rings1[wave];
     if (p.sk % BN || p.hd < D || p.hdv < D)  // chunks the loads leave out hold zeros
-        for (int i = lane * 8; i < 4 * TILE; i += 512) *reinterpret_cast<uint4 *>(ring + i) = make_uint4(0, 0, 0, 0);
+        for (int i = lane * 8; i < 2 * TILE; i += 512) {
+            *reinterpret_cast<uint4 *>(ring0 + i) = make_uint4(0, 0, 0, 0);
+            *reinterpret_cast<uint4 *>(ring1 + i) = make_uint4(0, 0, 0, 0);
+        }
 
     uint4 qf[DS];
 #pragma unroll
@@ -123,14 +123,11 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
     float m = -1e30f, l = 0.0f;
 
     __builtin_amdgcn_s_waitcnt(0xc07f);  // the zeros are written before a load can land on them
-    int stage = 0;
-    int64_t t = t0 + wave;
-    if (t < t1) load_pair32<D>(p, kp, vp, t * BN, ring, lane);
-    for (; t < t1; t += 4, stage ^= 1) {
+    auto tile = [&](int64_t t, const uint16_t *cur, uint16_t *next) __attribute__((always_inline)) {
         // tile t has landed; the other stage's reads were waited for by the MFMAs that used them
         __builtin_amdgcn_s_waitcnt(0x0f70);
-        if (t + 4 < t1) load_pair32<D>(p, kp, vp, (t + 4) * BN, ring + (stage ^ 1) * 2 * TILE, lane);
-        const char *Kb = reinterpret_cast<const char *>(ring + stage * 2 * TILE);
+        if (t + 4 < t1) load_pair32<D>(p, kp, vp, (t + 4) * BN, next, lane);
+        const char *Kb = reinterpret_cast<const char *>(cur);
         const char *Vb = Kb + TILE * 2;
         const int64_t k0 = t * BN;
         f32x16_t s;
@@ -140,14 +137,14 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
         for (int u = 0; u < DS; ++u)
             s = mfma32<F16>(*reinterpret_cast<const uint4 *>(Kb + kv_off<D>(l32, 16 * u + 8 * h)), qf[u], s);
         if (k0 + BN > full_end) {
-            const int64_t lim = min(CAUSAL ? qi + shift : p.sk - 1, p.sk - 1) - k0 - 4 * h;
+            const int lim = int(max(min(min(CAUSAL ? qi + shift : p.sk - 1, p.sk - 1) - k0 - 4 * h, int64_t(BN)), int64_t(-1)));
 #pragma unroll
             for (int e = 0; e < 16; ++e) s[e] = 8 * (e / 4) + (e % 4) <= lim ? s[e] : -INFINITY;
         }
         float mx = s[0];
 #pragma unroll
         for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;
+        mx = max_halves(mx) * c2;
         if (__any(mx > m + 8.0f)) {
             const float mnew = fmaxf(m, mx);
             const float alpha = fast_exp2(m - mnew);
@@ -183,6 +180,12 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
                 acc[dt] = mfma32<F16>(make_uint4(xa.x, xa.y, ya.x, ya.y), pb[t2], acc[dt]);
             }
         }
+    };
+    const int64_t first_tile = t0 + wave;
+    if (first_tile < t1) load_pair32<D>(p, kp, vp, first_tile * BN, ring0, lane);
+    for (int64_t t = first_tile; t < t1; t += 8) {
+        tile(t, ring0, ring1);
+        if (t + 4 < t1) tile(t + 4, ring1, ring0);
     }
     l += __shfl_xor(l, 32, 64);
 
@@ -193,7 +196,8 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
 #pragma unroll
     for (int w = 1; w < 4; ++w) top = fmaxf(top, ml[w][l32].x);
     const float own = fast_exp2(m - top);
-    float *red = reinterpret_cast<float *>(split_lds);  // [wave][row][D], chunks of 4 swizzled by row
+    static_assert(sizeof(rings0) >= 4 * 32 * D * sizeof(float), "the waves' sums fit the first stage");
+    float *red = reinterpret_cast<float *>(&rings0[0][0]);  // [wave][row][D], chunks of 4 swizzled by row
     if (qvalid) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -230,6 +234,11 @@ __global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitPar
         if (c == 0 && p.lse)
             p.lse[(b * p.heads + rn) * p.sq + ri] = tl > 0.0f ? (tm + __log2f(tl)) * 0.6931471805599453f : -INFINITY;
     }
+}
+
+template <int D, bool F16, bool CAUSAL>
+__global__ __launch_bounds__(256) void flash_split_kernel(AttnParams p, SplitParams sp) {
+    flash_split_body<D, F16, CAUSAL>(p, sp);
 }
 
 // A wave a query row: the splits' sums scaled to their common maximum and added in split order.
