@@ -460,12 +460,10 @@ __device__ __forceinline__ void load_row64_async(const float *src, int64_t k0, i
 // column a lane). Its adds are issued at the start of the next tile, so the wait for that tile's loads does
 // not also wait for adds just issued.
 template <int D> struct DkdvLds {
-    static constexpr int kTile = 64 * D;              // a Q or dO tile, elements
     static constexpr int kDsPitch = 128 + 8;          // dS row pitch (elements): rows on distinct banks
-    static constexpr int kBase = 4 * kTile;           // Q0 dO0 Q1 dO1
-    static constexpr int kAtomic = kBase + 128 * D + 64 * kDsPitch;  // + K (128 keys) + dS
+    static constexpr int kAtomic = 128 * D + 64 * kDsPitch;  // K (128 keys) + dS
     static constexpr int kStagePitch = 72;                           // STORE_DS staging row pitch (elements)
-    static constexpr int kStore = kBase + 4 * 32 * kStagePitch;      // + each wave's [32 keys][64 queries] dS
+    static constexpr int kStore = 4 * 32 * kStagePitch;              // each wave's [32 keys][64 queries] dS
 };
 
 // Whether a dK/dV workgroup takes a pair of causal key blocks.
@@ -478,10 +476,12 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
     constexpr int BM = 64;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int TILE = BM * D;
-    __shared__ __align__(1024) uint16_t smem[ATOMIC_DQ ? DkdvLds<D>::kAtomic : STORE_DS ? DkdvLds<D>::kStore : DkdvLds<D>::kBase];
-    __shared__ __align__(16) float Ls[2][BM];
-    __shared__ __align__(16) float Dl[2][BM];
-    uint16_t *const Ks = smem + DkdvLds<D>::kBase;    // ATOMIC_DQ: K rows [128][D], swizzled like a Q tile
+    // a stage's Q and dO tiles, LSE and delta are arrays of their own, so that reading one does not wait for the loads
+    // in flight into the other (flash_fwd_body)
+    __shared__ __align__(1024) uint16_t stage0[2 * TILE], stage1[2 * TILE];
+    __shared__ __align__(1024) uint16_t extra[ATOMIC_DQ ? DkdvLds<D>::kAtomic : STORE_DS ? DkdvLds<D>::kStore : 8];
+    __shared__ __align__(16) float Ls0[BM], Ls1[BM], Dl0[BM], Dl1[BM];
+    uint16_t *const Ks = extra;                       // ATOMIC_DQ: K rows [128][D], swizzled like a Q tile
     uint16_t *const dSb = Ks + 128 * D;               // ATOMIC_DQ: dS [64 queries][kDsPitch]
     (void)Ks;
     (void)dSb;
@@ -497,8 +497,10 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
     int64_t unit, pidx;
     xcd_order(int64_t(gridDim.x) / per, per, unit, pidx);
     const int64_t b = unit / p.kv_heads, nkv = unit % p.kv_heads;
-    zero_tiles(smem, ATOMIC_DQ ? DkdvLds<D>::kBase + 128 * D : DkdvLds<D>::kBase,
-               p.sq % BM || (ATOMIC_DQ && p.sk % 128) || p.hd < D || p.hdv < D);
+    const bool partial = p.sq % BM || (ATOMIC_DQ && p.sk % 128) || p.hd < D || p.hdv < D;
+    zero_tiles(stage0, 2 * TILE, partial);
+    zero_tiles(stage1, 2 * TILE, partial);
+    if (ATOMIC_DQ) zero_tiles(Ks, 128 * D, partial);
     for (int pass = 0; pass < (PAIR ? 2 : 1); ++pass) {
     const int64_t kblk = pass == 0 ? pidx : nkb - 1 - pidx;
     if (pass == 1) {
@@ -530,22 +532,21 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
         ls = lse2 + (b * p.heads + n) * p.sq;
         dl = p.delta + (b * p.heads + n) * p.sq;
     };
-    auto issue = [&](int j) {
+    auto issue = [&](int j, uint16_t *dst, float *lse_dst, float *delta_dst) __attribute__((always_inline)) {
         const uint16_t *qp, *gp;
         const float *ls, *dl;
         int64_t q0;
         tile_src(j, qp, gp, ls, dl, q0);
-        uint16_t *dst = smem + (j & 1) * 2 * TILE;
         load_tile_async<D>(qp, p.q_s, q0, p.sq, dst, wave, lane, p.hd);
         load_tile_async<D>(gp, p.do_s, q0, p.sq, dst + TILE, wave, lane, p.hdv);
-        if (wave == 0) load_row64_async(ls, q0, p.sq, Ls[j & 1], lane);
-        if (wave == 1) load_row64_async(dl, q0, p.sq, Dl[j & 1], lane);
+        if (wave == 0) load_row64_async(ls, q0, p.sq, lse_dst, lane);
+        if (wave == 1) load_row64_async(dl, q0, p.sq, delta_dst, lane);
     };
     if constexpr (ATOMIC_DQ) {  // waited for with the first tile's loads
         load_tile_async<D>(kp, p.k_s, kb0, p.sk, Ks, wave, lane, p.hd);
         load_tile_async<D>(kp, p.k_s, kb0 + 64, p.sk, Ks + 64 * D, wave, lane, p.hd);
     }
-    if (total > 0) issue(0);
+    if (total > 0) issue(0, stage0, Ls0, Dl0);
 
     // ATOMIC_DQ: this wave's dQ share of the previous tile, waiting to be added: NQ accumulators of 32 queries
     // x 32 head-dim columns (query half qh0 + c, columns 32 * dblk ...)
@@ -584,7 +585,8 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
         for (int e = 0; e < 16; ++e) adk[i][e] = adv[i][e] = 0.0f;
     const float c2 = p.scale * 1.4426950408889634f;
 
-    for (int j = 0; j < total; ++j) {
+    auto tile = [&](int j, const uint16_t *cur, const float *Lt, const float *Dt, uint16_t *next, float *next_lse,
+                    float *next_delta) __attribute__((always_inline)) {
         int64_t q0;
         {
             const uint16_t *qp, *gp;
@@ -597,10 +599,9 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
         else __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         flush_dq();  // the previous tile's dQ adds, ahead of this iteration's loads
-        if (j + 1 < total) issue(j + 1);
-        const char *Qb = reinterpret_cast<const char *>(smem + (j & 1) * 2 * TILE);
+        if (j + 1 < total) issue(j + 1, next, next_lse, next_delta);
+        const char *Qb = reinterpret_cast<const char *>(cur);
         const char *Gb = Qb + TILE * 2;
-        const float *Lt = Ls[j & 1], *Dt = Dl[j & 1];
         // rows q with q > sq - 1 or (causal) kj > q + shift are masked: tile row r is kept when rmin <= r < rmax
         // (with ATOMIC_DQ or STORE_DS also the key block past sk: its keys' P is zeroed)
         const bool masked = q0 + BM > p.sq || (CAUSAL && q0 + shift < kb0 + 127) ||
@@ -691,14 +692,17 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
             // + 16 half + 4 h); written into the wave's own LDS rows [32 keys][64 queries], they are read back
             // transposed (the B-operand read), each wave's two key steps x two query halves, and stored 16 bytes
             // a lane, 1 KiB contiguous an instruction. Masked rows and keys past sk hold zeros.
-            uint16_t *stg = smem + DkdvLds<D>::kBase + wave * (32 * DkdvLds<D>::kStagePitch);
+            uint16_t *stg = extra + wave * (32 * DkdvLds<D>::kStagePitch);
 #pragma unroll
             for (int qs = 0; qs < 2; ++qs)
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    uint16_t *row = stg + l32 * DkdvLds<D>::kStagePitch + 32 * qs + 16 * half + 4 * h;
-                    *reinterpret_cast<uint2 *>(row) = make_uint2(sb[qs][half].x, sb[qs][half].y);
-                    *reinterpret_cast<uint2 *>(row + 8) = make_uint2(sb[qs][half].z, sb[qs][half].w);
+                    // volatile: merged into one two-address write they would lose their array and wait for the
+                    // loads in flight
+                    typedef __attribute__((address_space(3))) volatile uint64_t lds_u64;
+                    lds_u64 *row = (lds_u64 *)(stg + l32 * DkdvLds<D>::kStagePitch + 32 * qs + 16 * half + 4 * h);
+                    row[0] = uint64_t(sb[qs][half].x) | (uint64_t(sb[qs][half].y) << 32);
+                    row[2] = uint64_t(sb[qs][half].z) | (uint64_t(sb[qs][half].w) << 32);
                 }
             const int64_t n_ = nkv * group + j / per_head;
             uint16_t *blk = p.ds + (((b * p.heads + n_) * nkb + kblk) * ((p.sq + 63) / 64) + q0 / 64) * (128 * 64);
@@ -810,6 +814,10 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
                 dq_left = p.sq - q0_;
             }
         }
+    };
+    for (int j = 0; j < total; j += 2) {
+        tile(j, stage0, Ls0, Dl0, stage1, Ls1, Dl1);
+        if (j + 1 < total) tile(j + 1, stage1, Ls1, Dl1, stage0, Ls0, Dl0);
     }
     if constexpr (ATOMIC_DQ) flush_dq();
     if (!kvalid) return;
@@ -873,7 +881,18 @@ __global__ __launch_bounds__(256, 2) void flash_dq_ds_kernel(AttnParams p) {
     constexpr int FN = D / 32;                                        // 32-column MFMA tiles of the head dim
     constexpr int KSTAGE = KT * D;                                    // K rows of a step in LDS, elements
     constexpr int KOPS = (64 / (1024 / (D * 2))) / 4;                 // K-row loads a lane a step
-    __shared__ __align__(1024) uint16_t smem[3 * KSTAGE];
+    // at head dim 64 three arrays, so that reading one stage does not wait for the loads in flight into the others
+    // (flash_fwd_body); at 128 their addresses would spill, which costs more (0.68 against 0.66 ms a backward of
+    // [8, 2048, 16, 128])
+    constexpr bool APART = D <= 64;
+    __shared__ __align__(1024) uint16_t stage0[APART ? KSTAGE : 3 * KSTAGE], stage1[APART ? KSTAGE : 8],
+        stage2[APART ? KSTAGE : 8];
+    auto stage = [&](auto bufc) __attribute__((always_inline)) -> uint16_t * {
+        constexpr int B = decltype(bufc)::value;
+        if constexpr (B == 0 || !APART) return stage0 + B * KSTAGE;
+        else if constexpr (B == 1) return stage1;
+        else return stage2;
+    };
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
     const int g = lane >> 4, s16 = lane & 15;
     const int64_t nqb = (p.sq + QB - 1) / QB;
@@ -894,8 +913,7 @@ __global__ __launch_bounds__(256, 2) void flash_dq_ds_kernel(AttnParams p) {
     uint4 fs[2][KS][2];
     // K rows of step kt into LDS stage B (three stages: issued two steps ahead)
     auto issue_k = [&](auto bufc, int kt) {
-        constexpr int B = decltype(bufc)::value;
-        load_tile_async<D, 4>(kp, p.k_s, int64_t(kt) * KT, p.sk, smem + B * KSTAGE, wave, lane, p.hd);
+        load_tile_async<D, 4>(kp, p.k_s, int64_t(kt) * KT, p.sk, stage(bufc), wave, lane, p.hd);
     };
     // dS fragments of step kt into register set B (two sets: issued one step ahead): 16-key steps 4 (kt & 1) + kk
     // and query halves qh of the 128-key block kt / 2
@@ -931,7 +949,7 @@ __global__ __launch_bounds__(256, 2) void flash_dq_ds_kernel(AttnParams p) {
         const bool live = qt < nqt && (!CAUSAL || (int64_t(kt) * KT <= qt * 64 + 63 + shift &&
                                                    qt >= max<int64_t>(0, int64_t(kt / 2) * 128 - shift) / 64));
         if (!live) return;
-        const char *ks_ = reinterpret_cast<const char *>(smem + BK * KSTAGE);
+        const char *ks_ = reinterpret_cast<const char *>(stage(bkc));
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) {
             const int krow = 16 * kk + 4 * h + s16 / 4;
@@ -947,7 +965,9 @@ __global__ __launch_bounds__(256, 2) void flash_dq_ds_kernel(AttnParams p) {
             }
         }
     };
-    zero_tiles(smem, 3 * KSTAGE, p.sk % KT || p.hd < D);
+    zero_tiles(stage(std::integral_constant<int, 0>{}), KSTAGE, p.sk % KT || p.hd < D);
+    zero_tiles(stage(std::integral_constant<int, 1>{}), KSTAGE, p.sk % KT || p.hd < D);
+    zero_tiles(stage(std::integral_constant<int, 2>{}), KSTAGE, p.sk % KT || p.hd < D);
     if (nk > 0) {
         issue_k(std::integral_constant<int, 0>{}, 0);
         issue_ds(std::integral_constant<int, 0>{}, 0);
