@@ -203,7 +203,8 @@ template <int NW, int D = 128> struct FwdOccupancy {
 
 // The two stages are arrays of their own, named by a constant in the loop below: were they halves of one array, every
 // LDS read would be taken to alias the loads just issued into the other half and wait for them (s_waitcnt vmcnt(0)
-// before the tile's first read), so that nothing overlapped.
+// before the tile's first read), so that nothing overlapped. [8, 2048, 16, 128] causal 243 -> 192-203 us (679-716
+// TFLOP/s), [2, 1777, 16 / 4, 64] 43 -> 37.
 template <int D, bool F16, bool CAUSAL, int NW>
 __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     constexpr int QB = 32 * NW;  // queries a workgroup
@@ -477,7 +478,7 @@ __global__ __launch_bounds__(256) void flash_dkdv_kernel(AttnParams p, const flo
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int TILE = BM * D;
     // a stage's Q and dO tiles, LSE and delta are arrays of their own, so that reading one does not wait for the loads
-    // in flight into the other (flash_fwd_body)
+    // in flight into the other (flash_fwd_body): the backward of [8, 2048, 16, 128] causal 0.70 -> 0.643 ms
     __shared__ __align__(1024) uint16_t stage0[2 * TILE], stage1[2 * TILE];
     __shared__ __align__(1024) uint16_t extra[ATOMIC_DQ ? DkdvLds<D>::kAtomic : STORE_DS ? DkdvLds<D>::kStore : 8];
     __shared__ __align__(16) float Ls0[BM], Ls1[BM], Dl0[BM], Dl1[BM];
