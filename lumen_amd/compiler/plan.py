@@ -1022,6 +1022,7 @@ class Plan:
     AUTOTUNE_MACS = 1 << 30
     AUTOTUNE_MARGIN = 0.03
     _tuned: dict = {}
+    _tuned_splits: dict = {}  # dots: the split count timed with the config
 
     def _apply_forced(self):
         """Configs of ``lumen_amd.autotune.use`` blocks: every plain GEMM step (any size) and every flash
@@ -1182,8 +1183,8 @@ class Plan:
                         # kernel run after run
                         if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
                             best, best_ms = (cfg, splits), ms
-                Plan._tuned[key] = best
-            st.config, st.splits = Plan._tuned[key]
+                Plan._tuned_splits[key], Plan._tuned[key] = best[1], best[0]
+            st.config, st.splits = Plan._tuned[key], Plan._tuned_splits[key]
 
     # Split-k policy: a bf16/f16 dot whose 256 x 256 output tiles cannot fill the 256 CUs is cut along k (in
     # powers of two, each part at least 1024 deep) until they do; its float32 partials live in the step's
