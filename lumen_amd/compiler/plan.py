@@ -598,16 +598,33 @@ class Plan:
                 if any(u != dv and pos.get(u, -1) >= si for u in lt.inputs):
                     continue  # an operand the loop reads is made after the dot
                 keep = dv in outputs or any(x != li for x in users.get(dv, []))
+                outs = ([dv] if keep else []) + list(lt.outputs)
+                try:  # past its first readers the loop may read the result at other elements (exp(y) + exp(y).t())
+                    self._epilogue_kernel(st, lt, lay, keep, outs).source()
+                except codegen.Unfusable:
+                    continue
                 st.epi = lt
                 st.epi_layout = lay
                 st.store_dot = keep
-                st.outputs = ([dv] if keep else []) + list(lt.outputs)
+                st.outputs = outs
                 st.inputs = list(st.inputs) + [u for u in lt.inputs if u != dv and u not in st.inputs]
                 st.nodes = list(st.nodes) + list(lt.nodes)
                 merged.add(li)
                 break
         self.steps = [st for i, st in enumerate(self.steps) if i not in merged]
         return bool(merged) | self._fuse_column_sums()
+
+    def _epilogue_kernel(self, st, loop, layout, store_dot, outputs, colsum=None, variant=0):
+        """The generated kernel of dot step ``st`` with ``loop`` in its store, over the values' present places."""
+        d, _ = self._gemm_desc(st.nodes[0])
+        views = {v: self.loc[v].view() for v in loop.inputs if v != st.nodes[0].output}
+        outs = {v: self.loc[v].view() for v in outputs}
+        if len(layout) == 2:
+            return codegen.SmallGemmEpilogueKernel(self.graph, st, loop, d, layout[1], store_dot, views, outs,
+                                                   aliased=self.aliased)
+        _, at, bt, f16 = layout
+        return codegen.GemmEpilogueKernel(self.graph, st, loop, d, at, bt, f16, store_dot, views, outs, colsum=colsum,
+                                          variant=variant, aliased=self.aliased)
 
     def _fuse_column_sums(self):
         """A float32 sum over the rows of a GEMM epilogue's [m, n] output that only the sum reads (a bias or
@@ -724,41 +741,24 @@ class Plan:
                 self.sources[si] = codegen.HEADER + body.replace("KNAME", name)
                 continue
             if st.kind == "dot" and getattr(st, "epi", None) is not None:
-                lin = [v for v in st.epi.inputs if v != st.nodes[0].output]
-                views = {v: self.loc[v].view() for v in lin}
-                outs = {v: self.loc[v].view() for v in st.outputs}
-                if len(st.epi_layout) == 2:
-                    d, _ = self._gemm_desc(st.nodes[0])
-                    k = codegen.SmallGemmEpilogueKernel(g, st, st.epi, d, st.epi_layout[1], st.store_dot, views, outs,
-                                                        aliased=self.aliased)
+                def kernel(variant=0):
+                    k = self._epilogue_kernel(st, st.epi, st.epi_layout, st.store_dot, st.outputs,
+                                              getattr(st, "epi_colsum", None), variant)
+                    k.far = far
                     body = k.source()
-                    k.name = st.name = f"gemm_{st.epi_layout[1][0]}_{hashlib.sha1(body.encode()).hexdigest()[:10]}"
-                    self.kernels[si] = k
-                    self.sources[si] = codegen.HEADER + body.replace("KNAME", k.name)
-                    continue
-                d, at, bt, f16 = st.epi_layout
-                d, _ = self._gemm_desc(st.nodes[0])
-                k = codegen.GemmEpilogueKernel(g, st, st.epi, d, at, bt, f16, st.store_dot, views, outs,
-                                               colsum=getattr(st, "epi_colsum", None), aliased=self.aliased)
-                k.far = far
-                body = k.source()
-                name = f"gemm_epi_{hashlib.sha1(body.encode()).hexdigest()[:10]}"
-                k.name = st.name = name
-                self.kernels[si] = k
-                self.sources[si] = codegen.HEADER + body.replace("KNAME", name)
+                    kind = f"gemm_{st.epi_layout[1][0]}" if len(st.epi_layout) == 2 else "gemm_epi"
+                    k.name = f"{kind}_{hashlib.sha1(body.encode()).hexdigest()[:10]}"
+                    return k, codegen.HEADER + body.replace("KNAME", k.name)
+
+                k, self.sources[si] = kernel()
+                self.kernels[si], st.name = k, k.name
                 # the other k loops, for the autotuner to time against this one (large dots whose operands and
                 # outputs do not overlap, so a timed run changes nothing the plan reads)
-                if config.compiler.autotune and d.m * d.n * d.k >= self.AUTOTUNE_MACS and not self._epi_overlaps(st):
+                if len(st.epi_layout) == 4 and config.compiler.autotune \
+                        and k.desc.m * k.desc.n * k.desc.k >= self.AUTOTUNE_MACS and not self._epi_overlaps(st):
                     for var in range(1, len(codegen.GemmEpilogueKernel.VARIANTS)):
-                        if not k.variant_ok(var):
-                            continue
-                        kv = codegen.GemmEpilogueKernel(g, st, st.epi, d, at, bt, f16, st.store_dot, views, outs,
-                                                        colsum=getattr(st, "epi_colsum", None), variant=var,
-                                                        aliased=self.aliased)
-                        kv.far = far
-                        bv = kv.source()
-                        kv.name = f"gemm_epi_{hashlib.sha1(bv.encode()).hexdigest()[:10]}"
-                        self.epi_alts.setdefault(si, []).append((var, kv, codegen.HEADER + bv.replace("KNAME", kv.name)))
+                        if k.variant_ok(var):
+                            self.epi_alts.setdefault(si, []).append((var, *kernel(var)))
                 continue
             if st.kind not in ("loop", "row", "reduce", "scatter_add"):
                 continue

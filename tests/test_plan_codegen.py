@@ -593,3 +593,36 @@ def test_split_counts_are_timed_where_the_dot_is_large():
     with L.config.compiler.patch(memory_limit=1 << 40):
         st = dot(512, 2048, 8192)
         assert st.split_choices == [st.splits] == [8]
+
+
+@pytest.mark.parametrize("m,k,n,dt", [(64, 64, 64, "float32"), (64, 64, 64, "bfloat16"), (16, 128, 16, "bfloat16"),
+                                      (4096, 64, 4096, "bfloat16")])
+def test_consumers_that_move_the_dots_result_keep_a_kernel_of_their_own(m, k, n, dt):
+    """A loop that applies an elementwise operation to a dot's result and then reads it at other elements (a transpose,
+    a reshape around one, a row or column of it) cannot run in the dot's store: it stays a loop, whatever kernel the
+    dot takes (the float32 fold, few rows, a streamed kernel). An elementwise consumer of the same dot still fuses,
+    through a reshape there and back too."""
+    def plan(consume, *more):
+        def fn(x, w, *rest):
+            return consume(F.matmul(x, w.t(), "float32", "float32"), *rest)
+
+        return _plan(fn, ((m, k), dt), ((n, k), dt), *more)
+
+    def swap(y):
+        return F.exp(y).reshape(m // 4, 4, n // 4, 4).transpose(1, 3).reshape(m, n) + 1.0
+
+    moving = [(lambda y: F.exp(y) + F.exp(y).t(),), (lambda y: F.exp(y).t() * 2.0,), (swap,),
+              (lambda y: F.exp(y) + F.exp(y)[:, :1],), (lambda y: F.exp(y) * F.exp(y)[1:2],),
+              (lambda y, b: F.relu(y + b) * F.relu(y + b).t(), ((n,), "float32"))]
+    for consume, *more in moving:
+        p = plan(consume, *more)
+        assert [st.kind for st in p.steps if st.kind != "view"] == ["dot", "loop"], [st.label() for st in p.steps]
+        assert getattr(p.steps[0], "epi", None) is None
+    symmetric = _plan(lambda x: (lambda e: (e + e.t()) * 0.5)(F.exp(F.matmul(x, x.t(), "float32", "float32") * 0.5)),
+                      ((m, k), dt))
+    assert [st.kind for st in symmetric.steps if st.kind != "view"] == ["dot", "loop"]
+    fused = [lambda y: F.exp(y) * 2.0 + F.tanh(y),
+             lambda y: (F.exp(y).reshape(m // 2, 2, n) * 2.0).reshape(m, n)]
+    for consume in fused:
+        p = plan(consume)
+        assert [st.kind for st in p.steps] == ["dot"] and p.steps[0].epi is not None
