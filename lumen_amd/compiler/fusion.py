@@ -16,7 +16,7 @@ other reduction is a reduce step of its own.
 from __future__ import annotations
 
 import math
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 
 from lumen_amd.graph.ir import ELEMENTWISE, Graph
 
@@ -563,7 +563,7 @@ def column_sums(graph, steps):
         space = (math.prod(x.shape[:-1]), x.shape[-1])
         if space[0] < COLSUM_MIN_ROWS or u in outputs or u not in pos or readers.get(u) != [st]:
             continue
-        made = steps[pos[u]]
+        made, moved = steps[pos[u]], []
         reader = min((steps.index(r) for r in readers.get(red.output, [])), default=len(steps))
         if made.kind == "row" and made.rows == space:
             row = made
@@ -580,18 +580,36 @@ def column_sums(graph, steps):
             if row is None:
                 continue
             have = {m.output for m in row.nodes}
-            row.nodes = sorted(row.nodes + [m for m in made.nodes if m.output not in have], key=lambda m: m.output)
-            gone.add(id(made))
+            moved = [m for m in made.nodes if m.output not in have]
         else:
             continue
-        row.colsums = row.colsums + [(u, red.output)]
-        row.outputs = [v for v in row.outputs if v != u] + [red.output]
-        row.scratch = len(row.colsums) * colsum_bytes(space)
-        row.inputs = _inputs_of(row.nodes)
+        nodes = sorted(row.nodes + moved, key=lambda m: m.output)
+        summing = replace(row, nodes=nodes, inputs=_inputs_of(nodes), colsums=row.colsums + [(u, red.output)],
+                          outputs=[v for v in row.outputs if v != u] + [red.output],
+                          scratch=(len(row.colsums) + 1) * colsum_bytes(space))
+        if not _row_kernel_ok(graph, summing):
+            continue
+        vars(row).update(vars(summing))
+        if made is not row:
+            gone.add(id(made))
         pos[red.output] = steps.index(row)
         gone.add(id(st))
     return _drop_unread(graph, [st for st in steps if id(st) not in gone])
 
+
+def _row_kernel_ok(graph, st):
+    """Whether a row kernel that sums columns can be generated for ``st`` (a row of one column has no column for the
+    generator to tell from the row)."""
+    from lumen_amd.compiler import codegen
+
+    def views(values):
+        return {v: codegen.View(t.dtype, t.shape, 0, codegen._contig(t.shape)) for v in values for t in [graph.types[v]]}
+
+    try:
+        codegen.LoopKernel(graph, st, "KNAME", views(st.inputs), views(st.outputs)).source()
+    except codegen.Unfusable:
+        return False
+    return True
 
 
 def colsum_bytes(space):

@@ -626,3 +626,17 @@ def test_consumers_that_move_the_dots_result_keep_a_kernel_of_their_own(m, k, n,
     for consume in fused:
         p = plan(consume)
         assert [st.kind for st in p.steps] == ["dot"] and p.steps[0].epi is not None
+
+
+@pytest.mark.parametrize("rows", [256, 1000])
+@pytest.mark.parametrize("cols", [1, 2, 8])
+def test_norms_of_few_columns_plan_with_their_weight_gradient(rows, cols):
+    """A norm's forward and backward over rows of few columns: the weight gradient's sum joins the row kernel where a
+    row kernel can read the summed value, and stays a step of its own over one column."""
+    def train(x, w, dy):
+        y, pull = L.vjp(lambda x, w: F.rms_norm(x.float(), x.size(-1), w.float()).bfloat16(), x, w)
+        return [y, *pull(dy)]
+
+    p = _plan(train, ((rows, cols), "bfloat16"), ((cols,), "bfloat16"), ((rows, cols), "bfloat16"))
+    row = next(st for st in p.steps if st.kind == "row")
+    assert len(row.colsums) == (cols > 1) and ("reduce" in [st.kind for st in p.steps]) == (cols == 1)
