@@ -5,6 +5,9 @@ from __future__ import annotations
 
 import contextlib
 import dataclasses
+import itertools
+
+_versions = itertools.count(1)
 
 
 @dataclasses.dataclass
@@ -46,7 +49,7 @@ class CompilerFlags:
     def __setattr__(self, name, value):
         object.__setattr__(self, name, value)
         if name != "_version":
-            object.__setattr__(self, "_version", self._version + 1)
+            object.__setattr__(self, "_version", next(_versions))  # never one seen before, whatever other threads set
 
     @contextlib.contextmanager
     def patch(self, **flags):
@@ -62,10 +65,11 @@ class CompilerFlags:
     def key(self):
         from lumen_amd import autotune
 
-        version, flags = self.__dict__.get("_flags", (None, None))
-        if version != self._version:  # setting any flag moves the version on
+        version = self._version  # setting any flag moves it on: read before the flags, as another thread may set one
+        known, flags = self.__dict__.get("_flags", (None, None))
+        if known != version:
             flags = tuple((f.name, getattr(self, f.name)) for f in dataclasses.fields(self) if f.name != "_version")
-            self.__dict__["_flags"] = (self._version, flags)
+            self.__dict__["_flags"] = (version, flags)
         return flags + (("forced", autotune.forced_key()),)
 
 

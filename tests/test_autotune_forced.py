@@ -38,3 +38,24 @@ def test_use_blocks_nest_and_key_plans():
     with pytest.raises(ValueError):
         with A.use(A.HipGemmConfig(0), A.HipGemmConfig(1)):
             pass
+
+
+def test_a_flag_set_while_the_plan_key_is_worked_out_is_in_the_next_key():
+    """Plan keys hold every flag as it is: one that another thread sets while a key is worked out (here: as its last
+    flag is read) is in the next key, not hidden behind the kept one."""
+    from lumen_amd.config import CompilerFlags
+
+    class Raced(CompilerFlags):
+        def __getattribute__(self, name):
+            value = super().__getattribute__(name)
+            if name == "fused_linear_cross_entropy_chunk_size" and super().__getattribute__("fuse"):
+                self.fuse = False
+            return value
+
+    flags = Raced()
+    flags.key()
+    assert dict(flags.key())["fuse"] is False
+    before = flags.key()
+    assert flags.key() == before
+    flags.autotune = False
+    assert flags.key() != before
