@@ -360,12 +360,6 @@ class Plan:
                 st.kind = "loop"
         self.loc: dict[int, Loc] = {}
         self.scratch: dict[int, Loc] = {}
-        self.in_place = self._in_place_outputs()
-        self.in_place_outputs = {g.outputs.index(v): i for v, i in self.in_place.items()}
-        self.aliased = frozenset(self.in_place) | frozenset(g.inputs[i] for i in self.in_place.values())
-        for i, v in enumerate(g.inputs):
-            t = g.types[v]
-            self.loc[v] = Loc(("in", i), 0, _contig(t.shape), t.dtype, t.shape)
         # a flash forward output read only through one transpose that keeps the head dim innermost (the
         # attention output going back to [B, S, N, H]) is written in the transposed order: the kernel takes
         # any strides, and the output projection then reads it in place instead of through a copy
@@ -379,11 +373,17 @@ class Plan:
                     if perm[-1] == len(perm) - 1:
                         o_perm[st.outputs[0]] = perm
         # such a transpose that the graph returns is fused as a copying loop: with the operand laid out its way
-        # it is a view like any other
+        # it is a view like any other (decided ahead of the in-place outputs, which only loops are)
         for st in self.steps:
             if st.kind == "loop" and len(st.nodes) == 1 and st.nodes[0].prim == "transpose" \
                     and o_perm.get(st.nodes[0].inputs[0]) == tuple(st.nodes[0].params["permutation"]):
                 st.kind = "view"
+        self.in_place = self._in_place_outputs()
+        self.in_place_outputs = {g.outputs.index(v): i for v, i in self.in_place.items()}
+        self.aliased = frozenset(self.in_place) | frozenset(g.inputs[i] for i in self.in_place.values())
+        for i, v in enumerate(g.inputs):
+            t = g.types[v]
+            self.loc[v] = Loc(("in", i), 0, _contig(t.shape), t.dtype, t.shape)
         # views first: resolved lazily in step order; a view that strides cannot express becomes a copy
         last_use: dict[int, int] = {}
         base_of: dict[int, int] = {}

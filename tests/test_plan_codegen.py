@@ -640,3 +640,14 @@ def test_norms_of_few_columns_plan_with_their_weight_gradient(rows, cols):
     p = _plan(train, ((rows, cols), "bfloat16"), ((cols,), "bfloat16"), ((rows, cols), "bfloat16"))
     row = next(st for st in p.steps if st.kind == "row")
     assert len(row.colsums) == (cols > 1) and ("reduce" in [st.kind for st in p.steps]) == (cols == 1)
+
+
+def test_a_returned_attention_output_is_no_in_place_update(monkeypatch):
+    """An attention output returned as a weight's new value is a view of the attention's own output: it is not marked
+    as written over the weight, in the first placement as little as in later ones, so the caller copies it back."""
+    args = [L.empty((2, 96, 4, 64), "bfloat16", "meta") for _ in range(3)]
+    g = L.make_graph(lambda q, k, v: (F.flash_attention(q, k, v, is_causal=True),))(*args)
+    monkeypatch.setattr(Plan, "_schedule", lambda self: self._place())  # one placement
+    p = Plan(g, "hip:0", build_kernels=False, donate={0: 0})
+    assert "loop" not in [st.kind for st in p.steps]
+    assert p.in_place_outputs == {} and p.output_locs[0].base == ("ws", 0) and p.output_locs[0].contiguous()
