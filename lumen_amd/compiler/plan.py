@@ -15,6 +15,7 @@ import math
 import struct
 from dataclasses import dataclass, replace
 
+from lumen_amd import autotune
 from lumen_amd import dtypes as D
 from lumen_amd import native as nv
 from lumen_amd.compiler import attention as attn_pass
@@ -540,7 +541,7 @@ class Plan:
         except NotImplementedError:
             return None
         small = _small_kind(d, ops)
-        if small is not None:
+        if small is not None and (small[0] == "fold" or autotune.forced(autotune.HipGemmConfig) is None):
             return d, small
         if d.a_dtype != d.b_dtype or d.a_dtype not in (nv.NHIP_BF16, nv.NHIP_F16) or d.k % 64 or d.n % 4:
             return None
@@ -1027,8 +1028,6 @@ class Plan:
     def _apply_forced(self):
         """Configs of ``lumen_amd.autotune.use`` blocks: every plain GEMM step (any size) and every flash
         forward step takes its family's forced config, untimed (``autotune/forced.rs``)."""
-        from lumen_amd import autotune
-
         gemm, attn = autotune.forced(autotune.HipGemmConfig), autotune.forced(autotune.HipAttentionConfig)
         for st in self.steps:
             if gemm is not None and st.kind == "dot" and getattr(st, "splits", 1) == 1 \

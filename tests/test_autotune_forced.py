@@ -59,3 +59,22 @@ def test_a_flag_set_while_the_plan_key_is_worked_out_is_in_the_next_key():
     assert flags.key() == before
     flags.autotune = False
     assert flags.key() != before
+
+
+def test_a_forced_gemm_config_reaches_few_row_dots_with_a_consumer():
+    """A dot of few rows whose consumer would run in its store is planned as a plain GEMM step inside a block that
+    forces a GEMM config, which it then takes; float32 dots, which have no configs, still fuse."""
+    import lumen_amd.functional as F
+    from lumen_amd.compiler.plan import Plan
+
+    def plan(dt):
+        args = [L.empty(s, dt, "meta") for s in ((16, 128), (64, 128))]
+        return Plan(L.make_graph(lambda x, w: F.relu(F.matmul(x, w.t(), "float32", "float32")))(*args), build_kernels=False)
+
+    assert [st.kind for st in plan("bfloat16").steps] == ["dot"]
+    with A.use(A.HipGemmConfig(0)):
+        p = plan("bfloat16")
+        assert [st.kind for st in p.steps] == ["dot", "loop"]
+        p._apply_forced()
+        assert p.steps[0].config == 0 and p.steps[0].forced
+        assert [st.kind for st in plan("float32").steps] == ["dot"]
