@@ -117,6 +117,17 @@ typedef struct {
 
 /* Queues D = A.B on the stream. A and B must be float dtypes of one kind (bf16/f16 together, or f32). */
 int nhip_gemm(const nhip_gemm_desc *desc, const void *a, const void *b, void *d);
+/* Which kernel nhip_gemm runs for `desc` over operands that both start on 16 bytes (`aligned`) or do not; nothing is
+ * queued. kernel[0] is the kind, kernel[1] and [2] the rows a wave (FOLD), the 16-row groups and the waves a workgroup
+ * (FEW_ROWS) or the tile config (TILED), else 0. For plans that generate the same kernel with another store. */
+enum {
+    NHIP_GEMM_EXACT = 0,     /* gemm_exact: operands of any strides */
+    NHIP_GEMM_FOLD = 1,      /* gemm_fold: float32 */
+    NHIP_GEMM_FEW_ROWS = 2,  /* gemm_skinny: 16-bit, at most 64 rows */
+    NHIP_GEMM_TILED = 3,     /* an MFMA tile config */
+    NHIP_GEMM_ANY = 4,       /* gemm_mfma over 16-bit rows of any length and alignment */
+};
+int nhip_gemm_kernel(const nhip_gemm_desc *desc, int aligned, int32_t kernel[3]);
 /* Number of tile configs nhip_gemm accepts in desc->config for bf16/f16 (autotuning, autotune/mod.rs). */
 int nhip_gemm_config_count(int *count);
 /* Split-k: D = A.B with k cut into desc->splits equal parts computed by separate workgroups (for shapes with

@@ -45,24 +45,12 @@ class Loc:
         return codegen.View(self.dtype, self.shape, self.offset, self.strides)
 
 
-def _mfma_layout(d) -> bool:
-    """Whether the MFMA kernels read a dot's operands (each k- or mn-contiguous with 16-byte aligned lines):
-    the host-side twin of kernels.hip's mfma_ready, without the pointer alignment."""
-    if d.a_k == 1 and d.k % 8 == 0 and (d.a_m % 8 == 0 or d.m == 1):
-        pass
-    elif not (d.a_m == 1 and d.m % 8 == 0 and d.a_k % 8 == 0):
-        return False
-    if d.b_k == 1 and d.k % 8 == 0 and (d.b_n % 8 == 0 or d.n == 1):
-        pass
-    elif not (d.b_n == 1 and d.n % 8 == 0 and d.b_k % 8 == 0):
-        return False
-    return all(d.a_batch[i] % 8 == 0 and d.b_batch[i] % 8 == 0 for i in range(d.nbatch))
-
-
-def _skinny(d) -> bool:
-    """Whether a dot in an MFMA layout runs as few rows by default: kernels.hip's skinny_default."""
-    groups = 1 if d.m <= 16 else 2 if d.m <= 32 else 4
-    return d.m <= 64 and d.a_k == 1 and d.b_k == 1 and groups * d.n <= 24576 and (groups <= 2 or d.k <= 2048)
+def _gemm_kernel(d, ops):
+    """``(kind, x, y)`` of the kernel nhip_gemm runs a dot as (nhip_gemm_kernel) over the places ``ops``."""
+    kernel = (C.c_int32 * 3)()
+    aligned = all(loc.offset * D.size_of(loc.dtype) % 16 == 0 for loc in ops[:2])
+    nv.call("nhip_gemm_kernel", C.byref(d), int(aligned), kernel)
+    return tuple(kernel)
 
 
 # float32 dots up to this many multiply-adds (15 us on the chip) take their consumer into the store: a launch and a
@@ -71,23 +59,14 @@ SMALL_FOLD_MACS = 1 << 27
 
 
 def _small_kind(d, ops):
-    """The SmallGemmEpilogueKernel ``kind`` nhip_gemm runs an unbatched dot as (kernels.hip: gemm_on's choice of
-    gemm_fold and its fold_rows, gemm_skinny's waves), or None where it takes another kernel."""
-    if not 0 < d.k < 1 << 30 or d.a_dtype != d.b_dtype:
-        return None
-    if d.a_dtype == NHIP_DT["float32"]:
-        if d.m * d.n * d.k > SMALL_FOLD_MACS:
-            return None
-        if (d.a_k != 1 and d.a_m != 1) or (d.b_k != 1 and d.b_n != 1):
-            return None
-        ak, rm = d.a_k == 1, 4 if d.a_k == 1 else 8
-        while rm > 1 and (d.m < rm or -(-d.m // rm) * -(-d.n // 64) < (2048 if ak else 1024)):
-            rm //= 2
-        return "fold", rm, ak, d.b_n == 1
-    if not _mfma_layout(d) or not _skinny(d) or any((loc.offset * D.size_of(loc.dtype)) % 16 for loc in ops[:2]):
-        return None
-    return "skinny", d.a_dtype == NHIP_DT["float16"], 1 if d.m <= 16 else 2 if d.m <= 32 else 4, \
-        8 if -(-d.n // 16) >= 512 else 16
+    """The SmallGemmEpilogueKernel ``kind`` of the kernel nhip_gemm runs an unbatched dot as, or None where that is
+    another."""
+    kind, x, y = _gemm_kernel(d, ops)
+    if kind == nv.NHIP_GEMM_FOLD and d.m * d.n * d.k <= SMALL_FOLD_MACS:
+        return "fold", x, d.a_k == 1, d.b_n == 1
+    if kind == nv.NHIP_GEMM_FEW_ROWS:
+        return "skinny", d.a_dtype == nv.NHIP_F16, x, y
+    return None
 
 
 def _contig(shape):
@@ -1201,7 +1180,7 @@ class Plan:
         the chip; whether that pays for writing and reading the partials depends on the shape: [8192, 2048] x [2048,
         512] takes 28 us whole and 36 in two parts, [2048, 8192] x [8192, 512] 78 and 41 in eight."""
         z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
-        if d.m * d.n * d.k * z < self.AUTOTUNE_MACS or -(-d.m // 256) * -(-d.n // 256) * z >= 256 or _skinny(d):
+        if d.m * d.n * d.k * z < self.AUTOTUNE_MACS or -(-d.m // 256) * -(-d.n // 256) * z >= 256:
             return [splits]
         s = [1]
         while s[-1] < self.SPLIT_MAX and d.k % (128 * s[-1]) == 0 and d.k // (2 * s[-1]) >= self.SPLIT_TUNED_MIN_K \
@@ -1214,12 +1193,10 @@ class Plan:
         if lhs.dtype not in ("bfloat16", "float16") or rhs.dtype != lhs.dtype:
             return 1, None
         try:
-            d, _ = self._gemm_desc(n)
+            d, ops = self._gemm_desc(n)
         except NotImplementedError:
             return 1, None
-        if not _mfma_layout(d) or any((loc.offset * D.size_of(loc.dtype)) % 16 for loc in (lhs, rhs)):
-            return 1, None
-        if _skinny(d):
+        if _gemm_kernel(d, ops)[0] != nv.NHIP_GEMM_TILED:
             return 1, None
         z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
         tiles = -(-d.m // 256) * -(-d.n // 256) * z

@@ -74,14 +74,16 @@ bool skinny_ok(const nhip_gemm_desc *d) {
     return d->m <= kSkinnyRows && d->a_k == 1 && d->b_k == 1 && d->k < (int64_t(1) << 30);
 }
 
-// Whether gemm_skinny is the default (plan.py's _skinny is the same rule). Every workgroup reads A's rows (in whole 16s,
+int skinny_groups(int64_t m) { return m <= 16 ? 1 : m <= 32 ? 2 : 4; }  // 16-row groups of A a wave takes
+
+// Whether gemm_skinny is the default. Every workgroup reads A's rows (in whole 16s,
 // 64 above 32) once, so many columns or many rows of a long k make those reads the larger part. Measured, us of
 // this and of the 128 x 128 kernel at its best split: [16, 2048] x [8192, 2048] 9.7, 17.4; [16, 8192] x [2048, 8192]
 // 16.4, 19.0; [16, 4096] x [1024, 4096] 9.5, 17.1; [32, 8192] x [2048, 8192] 23.7, 27.5; [64, 2048] x [4096, 2048]
 // 11.7, 18.2. Not: [16, 2048] x [32000, 2048] 37.4, 31.7; [64, 2048] x [8192, 2048] 20.6, 19.4; [64, 8192] x
 // [2048, 8192] 37.5, 19.8; [35, 3648] x [14592, 3648] 56.8, 51.7.
 bool skinny_default(const nhip_gemm_desc *d) {
-    const int64_t groups = d->m <= 16 ? 1 : d->m <= 32 ? 2 : 4;
+    const int64_t groups = skinny_groups(d->m);
     return skinny_ok(d) && groups * d->n <= 24576 && (groups <= 2 || d->k <= 2048);
 }
 
@@ -288,19 +290,23 @@ int launch_skinny_waves(hipStream_t st, const GemmShape &s, int64_t z, const voi
     return check(hipGetLastError(), "gemm_skinny launch");
 }
 
+int skinny_waves(int64_t n, int64_t z) { return (n + 15) / 16 * z >= 512 ? 8 : 16; }
+
 // 16 waves a workgroup where there are under two workgroups a CU ([16, 2048] x [8192, 2048], two a CU: 9.7 us with 8
 // waves, 11.7 with 16)
 template <bool F16, int MT>
 int launch_skinny_rows(hipStream_t st, const GemmShape &s, int64_t z, const void *a, const void *b, void *out, int dtype) {
-    if ((s.n + 15) / 16 * z >= 512) return launch_skinny_waves<F16, MT, 8>(st, s, z, a, b, out, dtype);
+    if (skinny_waves(s.n, z) == 8) return launch_skinny_waves<F16, MT, 8>(st, s, z, a, b, out, dtype);
     return launch_skinny_waves<F16, MT, 16>(st, s, z, a, b, out, dtype);
 }
 
 template <bool F16>
 int launch_skinny(hipStream_t st, const GemmShape &s, int64_t z, const void *a, const void *b, void *out, int dtype) {
-    if (s.m <= 16) return launch_skinny_rows<F16, 1>(st, s, z, a, b, out, dtype);
-    if (s.m <= 32) return launch_skinny_rows<F16, 2>(st, s, z, a, b, out, dtype);
-    return launch_skinny_rows<F16, 4>(st, s, z, a, b, out, dtype);
+    switch (skinny_groups(s.m)) {
+        case 1: return launch_skinny_rows<F16, 1>(st, s, z, a, b, out, dtype);
+        case 2: return launch_skinny_rows<F16, 2>(st, s, z, a, b, out, dtype);
+        default: return launch_skinny_rows<F16, 4>(st, s, z, a, b, out, dtype);
+    }
 }
 
 template <bool F16, bool AT, bool BT>
@@ -354,13 +360,14 @@ int launch_any(hipStream_t st, const GemmShape &s, int64_t z, const void *a, con
               : launch_any_layout<F16, false, false>(st, s, z, a, b, out, dtype);
 }
 
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+bool aligned16(const void *a, const void *b) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+}
 
 // Whether the MFMA kernel reads these operands: each k-contiguous or mn-contiguous, with 16-byte aligned
 // rows along its contiguous dimension. `at` / `bt` say an operand is mn-contiguous.
-bool mfma_ready(const nhip_gemm_desc *d, const void *a, const void *b, bool &at, bool &bt) {
-    if (d->a_dtype != d->b_dtype || d->a_dtype == NHIP_F32) return false;
-    if (!aligned16(a) || !aligned16(b)) return false;
+bool mfma_ready(const nhip_gemm_desc *d, bool aligned, bool &at, bool &bt) {
+    if (!aligned || d->a_dtype != d->b_dtype || d->a_dtype == NHIP_F32) return false;
     if (d->a_k == 1 && d->k % 8 == 0 && (d->a_m % 8 == 0 || d->m == 1)) at = false;
     else if (d->a_m == 1 && d->m % 8 == 0 && d->a_k % 8 == 0) at = true;
     else return false;
@@ -370,6 +377,29 @@ bool mfma_ready(const nhip_gemm_desc *d, const void *a, const void *b, bool &at,
     for (int i = 0; i < d->nbatch; ++i)
         if (d->a_batch[i] % 8 || d->b_batch[i] % 8) return false;
     return true;
+}
+
+// The kernel a dot runs as, over operands that both start on 16 bytes or do not. `at` / `bt`: the operand's contiguous
+// axis is m / n and not k.
+struct Choice {
+    int kind, config;
+    bool at, bt;
+};
+
+Choice choose(const nhip_gemm_desc *d, bool aligned) {
+    bool at = false, bt = false;
+    if (d->k <= 0) return {NHIP_GEMM_EXACT, -1, false, false};  // folds nothing: the exact kernel writes zeros
+    if (mfma_ready(d, aligned, at, bt)) {
+        const int cfg = d->config < 0 ? default_config(d) : d->config;
+        return {cfg == kSkinny ? NHIP_GEMM_FEW_ROWS : NHIP_GEMM_TILED, cfg, at, bt};
+    }
+    // operands contiguous along one axis each: 16-bit ones of any row length and alignment, and float32; others go
+    // through gemm_exact
+    if (d->a_dtype != d->b_dtype || (d->a_k != 1 && d->a_m != 1) || (d->b_k != 1 && d->b_n != 1))
+        return {NHIP_GEMM_EXACT, -1, false, false};
+    if (d->a_dtype != NHIP_F32) return {NHIP_GEMM_ANY, -1, d->a_k != 1, d->b_k != 1};
+    if (d->k < (int64_t(1) << 30)) return {NHIP_GEMM_FOLD, -1, d->a_k != 1, d->b_n == 1};
+    return {NHIP_GEMM_EXACT, -1, false, false};
 }
 
 }  // namespace
@@ -387,7 +417,7 @@ int gemm_splitk_on(hipStream_t st, const nhip_gemm_desc *d, const void *a, const
     if (d->m == 0 || d->n == 0 || z == 0) return 0;
     if (z > 65535 || d->splits > 64) return fail("nhip_gemm_splitk: more than 65535 batches or 64 splits");
     bool at = false, bt = false;
-    if (!mfma_ready(d, a, b, at, bt) || d->k % (64 * int64_t(d->splits)))
+    if (!mfma_ready(d, aligned16(a, b), at, bt) || d->k % (64 * int64_t(d->splits)))
         return fail("nhip_gemm_splitk: needs 16-bit operands in an MFMA layout and k a multiple of 64 * splits");
     if (!ws) return fail("nhip_gemm_splitk: no workspace");
     // partial products: contiguous [split][batch...][m][n]
@@ -434,9 +464,10 @@ int gemm_on(hipStream_t st, const nhip_gemm_desc *d, const void *a, const void *
     int64_t z = batch_count(d);
     if (d->m == 0 || d->n == 0 || z == 0) return 0;
     if (z > 65535) return fail("nhip_gemm: more than 65535 batches");
-    bool at = false, bt = false;
-    if (d->k > 0 && mfma_ready(d, a, b, at, bt)) {  // k == 0 folds nothing: the exact kernel writes zeros
-        int cfg = d->config < 0 ? default_config(d) : d->config;
+    const Choice c = choose(d, aligned16(a, b));
+    const bool f16 = d->a_dtype == NHIP_F16;
+    if (c.kind == NHIP_GEMM_TILED || c.kind == NHIP_GEMM_FEW_ROWS) {
+        const int cfg = c.config;
         if (cfg >= kNumConfigs) return fail("nhip_gemm: no tile config " + std::to_string(cfg));
         if (((cfg == kStream4w || cfg == kStream8w || cfg == kStream128 || cfg == kStreamPersist || cfg == kStream4w64X ||
               cfg == kStream8w64X) &&
@@ -444,28 +475,19 @@ int gemm_on(hipStream_t st, const nhip_gemm_desc *d, const void *a, const void *
             ((cfg == kStream8w32 || cfg == kStream8wX || cfg == kStream8wP || cfg == kStream4wX) && d->k % 32))
             return fail("nhip_gemm: the streamed configs need k to be a multiple of their k tile");
         if (cfg == kSkinny) {
-            if (!skinny_ok(d) || at || bt) return fail("nhip_gemm: config 16 takes at most 64 rows, both operands contiguous along k");
-            return d->a_dtype == NHIP_F16 ? launch_skinny<true>(st, s, z, a, b, out, d->d_dtype)
-                                          : launch_skinny<false>(st, s, z, a, b, out, d->d_dtype);
+            if (!skinny_ok(d) || c.at || c.bt) return fail("nhip_gemm: config 16 takes at most 64 rows, both operands contiguous along k");
+            return f16 ? launch_skinny<true>(st, s, z, a, b, out, d->d_dtype) : launch_skinny<false>(st, s, z, a, b, out, d->d_dtype);
         }
-        if (d->a_dtype == NHIP_F16) return launch_mfma<true>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
-        return launch_mfma<false>(st, cfg, s, z, a, b, out, d->d_dtype, at, bt);
+        return f16 ? launch_mfma<true>(st, cfg, s, z, a, b, out, d->d_dtype, c.at, c.bt)
+                   : launch_mfma<false>(st, cfg, s, z, a, b, out, d->d_dtype, c.at, c.bt);
     }
-    // operands contiguous along one axis each: 16-bit ones of any row length and alignment, and float32; others go
-    // through gemm_exact
-    if (d->a_dtype == d->b_dtype && d->a_dtype != NHIP_F32 && d->k > 0 && (d->a_k == 1 || d->a_m == 1) &&
-        (d->b_k == 1 || d->b_n == 1)) {
-        at = d->a_k != 1;
-        bt = d->b_k != 1;
-        return d->a_dtype == NHIP_F16 ? launch_any<true>(st, s, z, a, b, out, d->d_dtype, at, bt)
-                                      : launch_any<false>(st, s, z, a, b, out, d->d_dtype, at, bt);
-    }
-    if (d->a_dtype == NHIP_F32 && d->k > 0 && d->k < (int64_t(1) << 30) && (d->a_k == 1 || d->a_m == 1) &&
-        (d->b_k == 1 || d->b_n == 1)) {
+    if (c.kind == NHIP_GEMM_ANY)
+        return f16 ? launch_any<true>(st, s, z, a, b, out, d->d_dtype, c.at, c.bt)
+                   : launch_any<false>(st, s, z, a, b, out, d->d_dtype, c.at, c.bt);
+    if (c.kind == NHIP_GEMM_FOLD) {
         const float *fa = static_cast<const float *>(a), *fb = static_cast<const float *>(b);
-        if (d->a_k == 1)
-            return d->b_n == 1 ? launch_fold<true, true>(st, s, d, fa, fb, out) : launch_fold<true, false>(st, s, d, fa, fb, out);
-        return d->b_n == 1 ? launch_fold<false, true>(st, s, d, fa, fb, out) : launch_fold<false, false>(st, s, d, fa, fb, out);
+        if (!c.at) return c.bt ? launch_fold<true, true>(st, s, d, fa, fb, out) : launch_fold<true, false>(st, s, d, fa, fb, out);
+        return c.bt ? launch_fold<false, true>(st, s, d, fa, fb, out) : launch_fold<false, false>(st, s, d, fa, fb, out);
     }
     switch (d->d_dtype) {
         case NHIP_F32: return launch_exact<float>(st, s, d, a, b, out);
@@ -733,7 +755,7 @@ int lce_on(hipStream_t st, const nhip_lce_desc *d, const void *h, const void *w,
     if (!ws) return fail("nhip_linear_cross_entropy: no workspace");
     int64_t chunk = lce_chunk(d);
     if (lce_fused(d)) {
-        if (aligned16(h) && aligned16(w)) return lce_fused_on(st, d, h, w, target, out, ws);
+        if (aligned16(h, w)) return lce_fused_on(st, d, h, w, target, out, ws);
         // unaligned operands: the unfused form, as many rows a pass as the fused form's workspace holds
         const int64_t fit = int64_t(lce_workspace_bytes(d) / (size_t(d->v) * 4));
         chunk = chunk < fit ? chunk : fit;
@@ -775,6 +797,20 @@ int nhip_gemm(const nhip_gemm_desc *desc, const void *a, const void *b, void *d)
     hipStream_t s = stream_of_current();
     if (!s) return fail("no HIP stream: call nhip_set_device first");
     return gemm_on(s, desc, a, b, d);
+}
+
+int nhip_gemm_kernel(const nhip_gemm_desc *desc, int aligned, int32_t kernel[3]) {
+    if (desc->nbatch < 0 || desc->nbatch > 3) return fail("nhip_gemm: at most 3 batch axes");
+    const Choice c = choose(desc, aligned != 0);
+    kernel[0] = c.kind;
+    kernel[1] = kernel[2] = 0;
+    if (c.kind == NHIP_GEMM_TILED) kernel[1] = c.config;
+    if (c.kind == NHIP_GEMM_FOLD) kernel[1] = fold_rows(desc);
+    if (c.kind == NHIP_GEMM_FEW_ROWS) {
+        kernel[1] = skinny_groups(desc->m);
+        kernel[2] = skinny_waves(desc->n, batch_count(desc));
+    }
+    return 0;
 }
 
 int nhip_gemm_config_count(int *count) {

@@ -18,6 +18,7 @@ NHIP_F32, NHIP_BF16, NHIP_F16 = 0, 1, 2
 NHIP_BASE_WORKSPACE, NHIP_BASE_INPUT = 0, 1
 NHIP_STEP_GEMM, NHIP_STEP_FLASH_FWD, NHIP_STEP_FLASH_BWD, NHIP_STEP_COPY, NHIP_STEP_FILL, NHIP_STEP_LCE = 1, 2, 3, 4, 5, 6
 NHIP_LCE_I32, NHIP_LCE_I64 = 0, 1
+NHIP_GEMM_EXACT, NHIP_GEMM_FOLD, NHIP_GEMM_FEW_ROWS, NHIP_GEMM_TILED, NHIP_GEMM_ANY = range(5)
 
 
 class Props(C.Structure):
@@ -120,6 +121,7 @@ SIGNATURES = {
         C.c_int,
     ),
     "nhip_gemm": ([C.POINTER(GemmDesc), C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
+    "nhip_gemm_kernel": ([C.POINTER(GemmDesc), C.c_int, C.POINTER(C.c_int32)], C.c_int),
     "nhip_gemm_config_count": ([C.POINTER(C.c_int)], C.c_int),
     "nhip_gemm_splitk": ([C.POINTER(GemmDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nhip_gemm_workspace": ([C.POINTER(GemmDesc), C.POINTER(C.c_size_t)], C.c_int),

@@ -31,3 +31,25 @@ def test_device_count_without_a_gpu_is_an_answer():
     """nhip_device_count succeeds (0 devices where there is no GPU, as in the build container)."""
     n = native.device_count()
     assert n >= 0
+
+
+def test_gemm_kernel_says_what_nhip_gemm_would_run():
+    """Kinds by dtype, layout, alignment and forced config, with the parameters a generated store needs."""
+    def kernel(m, n, k, dt, a=None, b=None, aligned=True, config=-1):
+        d = native.GemmDesc(m=m, n=n, k=k, a_dtype=dt, b_dtype=dt, d_dtype=0, d_m=n, d_n=1, config=config)
+        (d.a_m, d.a_k), (d.b_k, d.b_n) = a or (k, 1), b or (1, k)
+        out = (C.c_int32 * 3)()
+        native.call("nhip_gemm_kernel", C.byref(d), int(aligned), out)
+        return tuple(out)
+
+    f32, bf16 = native.NHIP_F32, native.NHIP_BF16
+    assert kernel(256, 1024, 512, f32) == (native.NHIP_GEMM_FOLD, 2, 0)
+    assert kernel(256, 1024, 512, f32, aligned=False) == (native.NHIP_GEMM_FOLD, 2, 0)
+    assert kernel(256, 1024, 512, f32, a=(1024, 2))[0] == native.NHIP_GEMM_EXACT
+    assert kernel(16, 4096, 2048, bf16) == (native.NHIP_GEMM_FEW_ROWS, 1, 16)
+    assert kernel(64, 512, 2048, bf16, config=16) == (native.NHIP_GEMM_FEW_ROWS, 4, 16)
+    assert kernel(16, 4096, 2048, bf16, config=3) == (native.NHIP_GEMM_TILED, 3, 0)
+    assert kernel(16, 4096, 2048, bf16, aligned=False)[0] == native.NHIP_GEMM_ANY
+    assert kernel(4096, 4096, 4096, bf16)[0] == native.NHIP_GEMM_TILED
+    assert kernel(300, 5003, 511, bf16)[0] == native.NHIP_GEMM_ANY
+    assert kernel(300, 500, 0, bf16)[0] == native.NHIP_GEMM_EXACT
