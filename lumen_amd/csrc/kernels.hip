@@ -114,6 +114,21 @@ int fold_rows(const nhip_gemm_desc *d) {
     return 1;
 }
 
+// Whether gemm_fold is faster than gemm_exact, whose 64 x 64 tiles give a thread 16 sums: that reads A and B an eighth
+// as often, but leaves small results a few waves. `t` counts such tiles. Below k = 32 gemm_fold's pipeline never
+// fills; above, A contiguous along m (a scalar load a k) and B along n (unaligned 16-byte loads) need a longer k to
+// pay on results of many tiles. Measured, us of gemm_exact and gemm_fold: both operands along k, 1024^2 (256 tiles),
+// k = 31: 7.7, 10.4; 32: 8.2, 6.3; 2048^2, 40: 17.4, 21.3; 96: 31.5, 26.4; 8192 x 4096, 31: 59.5, 195. B along n: 8192^2,
+// 256: 752, 763; 512: 1476, 1461. A along m too: 2048^2, 64: 18.6, 22.0; 512: 121, 111; 8192 x 4096, 1000: 1357, 1480.
+bool fold_better(const nhip_gemm_desc *d) {
+    const int64_t t = (d->m + 63) / 64 * ((d->n + 63) / 64) * batch_count(d);
+    const bool ak = d->a_k == 1, bn = d->b_n == 1;
+    if (ak ? t <= 128 : t < 128) return true;
+    if (d->k < 32) return false;
+    if (t < 1024) return ak || t < 512 || d->k >= 64;
+    return d->k >= (!ak ? t / 4 : bn ? t / 16 : 96);
+}
+
 template <int RM, bool AK, bool BN>
 int launch_fold_rows(hipStream_t st, GemmShape s, const nhip_gemm_desc *d, const float *a, const float *b, void *out) {
     s.tiles_m = int((s.m + 4 * RM - 1) / (4 * RM));
@@ -393,12 +408,12 @@ Choice choose(const nhip_gemm_desc *d, bool aligned) {
         const int cfg = d->config < 0 ? default_config(d) : d->config;
         return {cfg == kSkinny ? NHIP_GEMM_FEW_ROWS : NHIP_GEMM_TILED, cfg, at, bt};
     }
-    // operands contiguous along one axis each: 16-bit ones of any row length and alignment, and float32; others go
-    // through gemm_exact
+    // operands contiguous along one axis each: 16-bit ones of any row length and alignment, and float32 where that is
+    // faster; others go through gemm_exact
     if (d->a_dtype != d->b_dtype || (d->a_k != 1 && d->a_m != 1) || (d->b_k != 1 && d->b_n != 1))
         return {NHIP_GEMM_EXACT, -1, false, false};
     if (d->a_dtype != NHIP_F32) return {NHIP_GEMM_ANY, -1, d->a_k != 1, d->b_k != 1};
-    if (d->k < (int64_t(1) << 30)) return {NHIP_GEMM_FOLD, -1, d->a_k != 1, d->b_n == 1};
+    if (d->k < (int64_t(1) << 30) && fold_better(d)) return {NHIP_GEMM_FOLD, -1, d->a_k != 1, d->b_n == 1};
     return {NHIP_GEMM_EXACT, -1, false, false};
 }
 

@@ -251,6 +251,29 @@ def test_float32_fold_is_bit_exact_in_every_layout(hip, at, bt, m, n, k, z, out)
         assert np.array_equal(got[ok], bits[ok]) and ok.sum() >= (m - 1) * n
 
 
+@pytest.mark.parametrize("at,bt", [(False, True), (False, False), (True, True), (True, False)])
+@pytest.mark.parametrize("m,n", [(1030, 1000), (1025, 2050), (1, 8000)])
+def test_float32_kernels_agree_on_both_sides_of_the_choice(hip, at, bt, m, n):
+    """Short and longer k over one result, where the library goes from gemm_exact to gemm_fold: each the sequential
+    fold, bit for bit."""
+    rng = np.random.default_rng(m + n)
+    kinds = set()
+    for k in (1, 31, 32, 65, 160):
+        a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+        want = np.zeros((m, n), np.float32)
+        for i in range(k):
+            want += a[:, i, None] * b[i]
+        da, db = Dev(np.ascontiguousarray(a.T) if at else a), Dev(b if bt else np.ascontiguousarray(b.T))
+        dd = Dev(nbytes=m * n * 4)
+        desc = _desc(m, n, k, 1 if at else k, m if at else 1, n if bt else 1, 1 if bt else k, dt=nv.NHIP_F32, out=nv.NHIP_F32)
+        kind = (C.c_int32 * 3)()
+        nv.call("nhip_gemm_kernel", C.byref(desc), 1, kind)
+        kinds.add(kind[0])
+        nv.call("nhip_gemm", C.byref(desc), da.ptr, db.ptr, dd.ptr)
+        np.testing.assert_array_equal(dd.get((m, n), np.float32), want)
+    assert kinds == ({nv.NHIP_GEMM_EXACT, nv.NHIP_GEMM_FOLD} if m > 1 else {nv.NHIP_GEMM_FOLD})
+
+
 @pytest.mark.parametrize("m,n,k,z,out,dt", [
     (1, 1, 8, 1, nv.NHIP_F32, nv.NHIP_BF16), (1, 17, 64, 1, nv.NHIP_F32, nv.NHIP_F16), (3, 8200, 512, 1, nv.NHIP_F32, nv.NHIP_BF16),
     (16, 100, 1032, 2, nv.NHIP_BF16, nv.NHIP_BF16), (17, 640, 2120, 1, nv.NHIP_F32, nv.NHIP_F16),

@@ -46,6 +46,12 @@ def test_gemm_kernel_says_what_nhip_gemm_would_run():
     assert kernel(256, 1024, 512, f32) == (native.NHIP_GEMM_FOLD, 2, 0)
     assert kernel(256, 1024, 512, f32, aligned=False) == (native.NHIP_GEMM_FOLD, 2, 0)
     assert kernel(256, 1024, 512, f32, a=(1024, 2))[0] == native.NHIP_GEMM_EXACT
+    for m, n, k, a, b, kind in [(8192, 4096, 31, None, None, "EXACT"), (8192, 4096, 96, None, None, "FOLD"),
+                                (1024, 1024, 31, None, None, "EXACT"), (1024, 1024, 32, None, None, "FOLD"),
+                                (512, 1024, 1, None, None, "FOLD"), (8192, 8192, 256, None, (8192, 1), "EXACT"),
+                                (4096, 4096, 256, None, (4096, 1), "FOLD"), (8192, 4096, 1000, (1, 8192), (4096, 1), "EXACT"),
+                                (1024, 1024, 40, (1, 1024), (1024, 1), "FOLD"), (512, 1024, 16, (1, 512), None, "EXACT")]:
+        assert kernel(m, n, k, f32, a, b)[0] == getattr(native, f"NHIP_GEMM_{kind}"), (m, n, k)
     assert kernel(16, 4096, 2048, bf16) == (native.NHIP_GEMM_FEW_ROWS, 1, 16)
     assert kernel(64, 512, 2048, bf16, config=16) == (native.NHIP_GEMM_FEW_ROWS, 4, 16)
     assert kernel(16, 4096, 2048, bf16, config=3) == (native.NHIP_GEMM_TILED, 3, 0)
