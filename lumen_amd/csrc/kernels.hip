@@ -76,15 +76,21 @@ bool skinny_ok(const nhip_gemm_desc *d) {
 
 int skinny_groups(int64_t m) { return m <= 16 ? 1 : m <= 32 ? 2 : 4; }  // 16-row groups of A a wave takes
 
-// Whether gemm_skinny is the default. Every workgroup reads A's rows (in whole 16s,
-// 64 above 32) once, so many columns or many rows of a long k make those reads the larger part. Measured, us of
-// this and of the 128 x 128 kernel at its best split: [16, 2048] x [8192, 2048] 9.7, 17.4; [16, 8192] x [2048, 8192]
-// 16.4, 19.0; [16, 4096] x [1024, 4096] 9.5, 17.1; [32, 8192] x [2048, 8192] 23.7, 27.5; [64, 2048] x [4096, 2048]
-// 11.7, 18.2. Not: [16, 2048] x [32000, 2048] 37.4, 31.7; [64, 2048] x [8192, 2048] 20.6, 19.4; [64, 8192] x
-// [2048, 8192] 37.5, 19.8; [35, 3648] x [14592, 3648] 56.8, 51.7.
+// Whether gemm_skinny is the default. A workgroup takes 16 columns and reads all of its batch's A rows (in whole 16s, 64
+// above 32), so many columns (over the batch), many rows of a long k or large A's make those reads the larger part.
+// Measured, us of this and of the tiled kernels at their best split ([m, k] x [n, k]): [16, 2048] x [8192, 2048] 9.4, 17.6;
+// [16, 8192] x [2048, 8192] 16.4, 19.0 (weights out of the caches 18.6, 23.5); [32, 4096] x [4096, 4096] 13.2, 18.5; [64, 2048] x
+// [4096, 2048] 11.7, 15.1; 16 of [16, 1024] x [512, 1024] 6.3, 12.3; 64 of [1, 1024] x [1024, 1024] 23.8, 29.9. Not: [16, 4096] x
+// [16384, 4096] 30.2, 25.9; [16, 2048] x [32000, 2048] 37.4, 31.7; [32, 8192] x [2048, 8192] 23.6, 19.2; [64, 4096] x [2048, 4096]
+// 20.4, 14.4; 64 of [16, 64] x [512, 64] 5.4, 4.3; 64 of [64, 64] x [2048, 64] 49.1, 15.5; 64 of [64, 1024] x [64, 1024] 14.1, 11.0.
 bool skinny_default(const nhip_gemm_desc *d) {
-    const int64_t groups = skinny_groups(d->m);
-    return skinny_ok(d) && groups * d->n <= 24576 && (groups <= 2 || d->k <= 2048);
+    if (!skinny_ok(d)) return false;
+    const int64_t groups = skinny_groups(d->m), z = batch_count(d), columns = z * d->n;
+    if (z * d->m * d->k > (groups == 1 ? 1 << 22 : 1 << 21)) return false;
+    if (groups * columns > 24576) return d->m == 1 && z > 1 && d->k >= 128;
+    if (groups == 1) return columns * d->k <= 1 << 25 && (d->k <= 4096 || (d->k <= 8192 && (d->m <= 8 || columns >= 2048)));
+    if (groups == 2) return columns * d->k <= 1 << 24 && d->k <= 4096;
+    return d->k <= 2048;
 }
 
 // The default tile for a shape: the streamed 256 x 256 kernel when k allows it and its tiles fill the 256 CUs,

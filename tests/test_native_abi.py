@@ -35,8 +35,9 @@ def test_device_count_without_a_gpu_is_an_answer():
 
 def test_gemm_kernel_says_what_nhip_gemm_would_run():
     """Kinds by dtype, layout, alignment and forced config, with the parameters a generated store needs."""
-    def kernel(m, n, k, dt, a=None, b=None, aligned=True, config=-1):
-        d = native.GemmDesc(m=m, n=n, k=k, a_dtype=dt, b_dtype=dt, d_dtype=0, d_m=n, d_n=1, config=config)
+    def kernel(m, n, k, dt, a=None, b=None, aligned=True, config=-1, z=1):
+        d = native.GemmDesc(m=m, n=n, k=k, a_dtype=dt, b_dtype=dt, d_dtype=0, d_m=n, d_n=1, config=config, nbatch=1)
+        d.batch[0], d.a_batch[0], d.b_batch[0], d.d_batch[0] = z, m * k, n * k, m * n
         (d.a_m, d.a_k), (d.b_k, d.b_n) = a or (k, 1), b or (1, k)
         out = (C.c_int32 * 3)()
         native.call("nhip_gemm_kernel", C.byref(d), int(aligned), out)
@@ -53,6 +54,13 @@ def test_gemm_kernel_says_what_nhip_gemm_would_run():
                                 (1024, 1024, 40, (1, 1024), (1024, 1), "FOLD"), (512, 1024, 16, (1, 512), None, "EXACT")]:
         assert kernel(m, n, k, f32, a, b)[0] == getattr(native, f"NHIP_GEMM_{kind}"), (m, n, k)
     assert kernel(16, 4096, 2048, bf16) == (native.NHIP_GEMM_FEW_ROWS, 1, 16)
+    few = [(16, 8192, 2048, 1), (16, 2048, 8192, 1), (8, 512, 8192, 1), (32, 4096, 4096, 1), (64, 4096, 2048, 1), (16, 512, 1024, 16),
+           (16, 256, 128, 64), (1, 1024, 1024, 64)]
+    tiled = [(16, 16384, 4096, 1), (16, 512, 8192, 1), (16, 32000, 2048, 1), (32, 2048, 8192, 1), (64, 2048, 4096, 1), (16, 512, 64, 64),
+             (64, 2048, 64, 64), (64, 64, 1024, 64), (32, 512, 128, 64), (8, 512, 64, 64), (65, 512, 512, 1)]
+    for cases, kind in ((few, native.NHIP_GEMM_FEW_ROWS), (tiled, native.NHIP_GEMM_TILED)):
+        for m, n, k, z in cases:
+            assert kernel(m, n, k, bf16, z=z)[0] == kind, (m, n, k, z)
     assert kernel(64, 512, 2048, bf16, config=16) == (native.NHIP_GEMM_FEW_ROWS, 4, 16)
     assert kernel(16, 4096, 2048, bf16, config=3) == (native.NHIP_GEMM_TILED, 3, 0)
     assert kernel(16, 4096, 2048, bf16, aligned=False)[0] == native.NHIP_GEMM_ANY
