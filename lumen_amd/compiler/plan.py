@@ -53,16 +53,13 @@ def _gemm_kernel(d, ops):
     return tuple(kernel)
 
 
-# float32 dots up to this many multiply-adds (15 us on the chip) take their consumer into the store: a launch and a
-# pass over the result are a tenth of such a call or more ([256, 512] x [512, 1024] with its relu: 15.5 -> 11.6 us)
-SMALL_FOLD_MACS = 1 << 27
-
-
 def _small_kind(d, ops):
     """The SmallGemmEpilogueKernel ``kind`` of the kernel nhip_gemm runs an unbatched dot as, or None where that is
-    another."""
+    another. A fold takes its consumer at every size: a launch and a pass over the result less, in us with relu apart
+    and in the store: [256, 512] x [512, 1024] 16.2, 12.2; [257, 512] 19.3, 15.4; [1024, 512] x [512, 1024] 34.8, 28.9; [4096,
+    1024] x [1024, 4096] 737, 680, and 787, 607 where both operands are contiguous along m and n."""
     kind, x, y = _gemm_kernel(d, ops)
-    if kind == nv.NHIP_GEMM_FOLD and d.m * d.n * d.k <= SMALL_FOLD_MACS:
+    if kind == nv.NHIP_GEMM_FOLD:
         return "fold", x, d.a_k == 1, d.b_n == 1
     if kind == nv.NHIP_GEMM_FEW_ROWS:
         return "skinny", d.a_dtype == nv.NHIP_F16, x, y

@@ -651,3 +651,9 @@ def test_a_returned_attention_output_is_no_in_place_update(monkeypatch):
     p = Plan(g, "hip:0", build_kernels=False, donate={0: 0})
     assert "loop" not in [st.kind for st in p.steps]
     assert p.in_place_outputs == {} and p.output_locs[0].base == ("ws", 0) and p.output_locs[0].contiguous()
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 1024, 512), (257, 1024, 512), (1024, 1024, 512), (4096, 4096, 1024)])
+def test_float32_folds_take_their_consumer_at_every_size(m, n, k):
+    p = _plan(lambda x, w: F.relu(F.matmul(x, w, "float32", "float32")), ((m, k), "float32"), ((k, n), "float32"))
+    assert [st.kind for st in p.steps] == ["dot"] and p.steps[0].epi_layout[1][0] == "fold"
