@@ -219,8 +219,28 @@ class Plan:
         for n in self.graph.nodes:
             if n.prim == "concatenate" and n.params["dimension"] == 0 and tuple(n.inputs) in packed_inputs:
                 self.packed.add(n.output)
+        self._lay_out_steps()
+        limit = config.compiler.memory_limit
+        if limit and self.workspace_bytes > limit and config.compiler.schedules:
+            # the schedules were compared before dots took their consumers into their stores: again, with them there
+            sizes = {self.schedule: self.workspace_bytes}
+            for name in schedule.SCHEDULES:
+                if name not in sizes:
+                    self._lay_out_steps(name)
+                    sizes[name] = self.workspace_bytes
+            self._lay_out_steps(min(sizes, key=sizes.get))
+
+    def _lay_out_steps(self, order=None):
+        """Steps in schedule ``order`` (``"fused"`` or one of ``schedule.SCHEDULES``; by default the one whose
+        placement needs the least workspace), placed, dots with the consumers their stores take."""
         self.steps = self._fuse()
-        self._schedule()
+        if order is None:
+            self._schedule()
+        else:
+            self.schedule = order
+            if order != "fused":
+                self.steps = schedule.SCHEDULES[order](self.graph, self.steps)
+            self._place()
         if config.compiler.fuse and config.compiler.epilogue_fusion and self._fuse_epilogues():
             self._place()
 
