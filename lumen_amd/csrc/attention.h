@@ -196,9 +196,11 @@ __device__ __forceinline__ void load_tile_async(const uint16_t *src, int64_t rs,
 // Workgroup sizes of the forward kernel (the attention tile configs): NW waves of 32 queries each share every
 // K/V tile a workgroup streams through LDS. More waves read K and V fewer times per query; fewer fill the CUs
 // when there are few query blocks. Two workgroups a CU hold the 64 KiB (D = 128) double-buffered tiles, so
-// each wave keeps 256 VGPRs at 4 waves a workgroup and 8 (one workgroup a CU at 8).
+// each wave keeps 256 VGPRs at 4 waves a workgroup and 8 (one workgroup a CU at 8). At D = 64 a wave is held to 168
+// VGPRs, three waves a SIMD: left to itself a causal one takes 172 and two ([32, 1000, 16, 64] 164 us, 138 with three;
+// [8, 2048, 16, 64] 132, 117; [32, 512, 32 / 8, 64] 110, 92). Four spill 24 registers (173, 129, 108).
 template <int NW, int D = 128> struct FwdOccupancy {
-    static constexpr int kBlocks = D > 128 ? 1 : (NW >= 8 ? 1 : (NW >= 4 ? 2 : 4));
+    static constexpr int kBlocks = D > 128 ? 1 : NW >= 8 ? 1 : NW >= 4 ? (D > 64 ? 2 : 3) : 4;
 };
 
 // The two stages are arrays of their own, named by a constant in the loop below: were they halves of one array, every
@@ -1185,7 +1187,7 @@ inline nhipk::AttnParams attn_params(const nhip_attn_desc *d) {
     return p;
 }
 
-// The forward's tile configs (nhip_attn_desc.config; -1 is config 0): 0 = 4 waves (128 queries) a
+// The forward's tile configs (nhip_attn_desc.config; -1 picks, launch_fwd): 0 = 4 waves (128 queries) a
 // workgroup, 1 = 8 waves (256 queries), 2 = 2 waves (64 queries). The backward kernels have one tile each.
 constexpr int kNumAttnConfigs = 3;
 
@@ -1237,7 +1239,10 @@ int launch_fwd(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *
         // head dim 256: 4 waves, one workgroup a CU (its K/V tiles fill 128 KiB of LDS), whatever the config
         return launch_fwd_nw<D, F16, CAUSAL, 4>(s, p, d);
     } else {
-        switch (d->config < 0 ? 0 : d->config) {
+        // by default 128 queries a workgroup, or 64 at head dim 64 where there are no more: waves without a query
+        // hold registers that others could use ([32, 1, 32 / 8, 64] over 1 key 8.9 us, 6.6; over 65 11.6, 7.8; 64 queries
+        // over 256 keys 18.9, 16.9)
+        switch (d->config >= 0 ? d->config : D == 64 && d->sq <= 64 ? 2 : 0) {
             case 1: return launch_fwd_nw<D, F16, CAUSAL, 8>(s, p, d);
             case 2: return launch_fwd_nw<D, F16, CAUSAL, 2>(s, p, d);
             default: return launch_fwd_nw<D, F16, CAUSAL, 4>(s, p, d);

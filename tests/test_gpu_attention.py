@@ -351,3 +351,21 @@ def test_forward_with_keys_divided_over_waves(hip, case, workspace):
     assert np.abs(got - want).max() <= 4 * tol * np.abs(want).max()
     np.testing.assert_allclose(lse.get((b, n, sq), np.float32), (top + np.log(e.sum(-1, keepdims=True)))[..., 0],
                                rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("sq,sk,d,causal", [(1, 1, 64, True), (40, 65, 64, True), (64, 64, 48, False), (65, 65, 64, True)])
+def test_default_forward_tile_gives_the_configs_bits(hip, sq, sk, d, causal):
+    """The workgroup size the forward picks by itself (64 queries up to 64 of them, else 128) changes no bit."""
+    b, n = 64, 8  # enough heads that the keys are not divided
+    rng = np.random.default_rng(sq)
+    q, k, v = (D.bf16_bits(rng.standard_normal(s).astype(np.float32)) for s in ((b, sq, n, d), (b, sk, n, d), (b, sk, n, d)))
+    desc = attn_desc(b, sq, sk, n, n, d, causal, 1.0 / math.sqrt(d))
+    dq, dk, dv, o, lse = Dev(q), Dev(k), Dev(v), Dev(nbytes=q.nbytes), Dev(nbytes=b * n * sq * 4)
+    got = []
+    for config in (-1, 0, 2):
+        desc.config = config
+        nv.call("nhip_flash_fwd", C.byref(desc), dq.ptr, dk.ptr, dv.ptr, o.ptr, lse.ptr)
+        got.append((o.get(q.shape, np.uint16), lse.get((b, n, sq), np.uint32)))
+    for x in got[1:]:
+        np.testing.assert_array_equal(x[0], got[0][0])
+        np.testing.assert_array_equal(x[1], got[0][1])
