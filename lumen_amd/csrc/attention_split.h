@@ -78,9 +78,15 @@ __device__ __forceinline__ void flash_split_body(const AttnParams &p, const Spli
     __shared__ float2 ml[4][32];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, l32 = lane & 31, g = lane >> 4, s16 = lane & 15;
-    // the workgroups of a unit (batch, key/value head, row tile) are consecutive, the row tiles of a head too
-    const int64_t unit = blockIdx.x / sp.splits, split = blockIdx.x % sp.splits;
-    const int64_t rt = unit % sp.tiles, head = unit / sp.tiles;
+    // The workgroups of a (batch, key/value head) run on one XCD, whose L2 then holds the keys its row tiles share: 32 x 8
+    // heads of 64, 256 rows, 4096 keys 291 us spread over the XCDs, 153 (7 TB/s of K and V read again); 8 x 16 heads, 200
+    // rows 133, 61. As xcd_order, in 32-bit scalars: from vector values the addresses would put each load into a loop
+    // over the lanes.
+    const uint32_t heads = uint32_t(p.batch * p.kv_heads), per = uint32_t(sp.tiles * sp.splits), wg = blockIdx.x;
+    const uint32_t at = heads % 8 ? wg : (wg / 8 / per * 8 + wg % 8) * per + wg / 8 % per;
+    const int64_t head = __builtin_amdgcn_readfirstlane(at / per);
+    const int64_t rt = __builtin_amdgcn_readfirstlane(at % per / uint32_t(sp.splits));
+    const int64_t split = __builtin_amdgcn_readfirstlane(at % uint32_t(sp.splits)), unit = head * sp.tiles + rt;
     const int64_t b = head / p.kv_heads, nkv = head % p.kv_heads;
     const int64_t row = rt * 32 + l32, group = p.heads / p.kv_heads;
     const int live = int(min(int64_t(32), sp.rows - rt * 32));  // rows of this tile

@@ -315,16 +315,26 @@ def test_partial_tiles_ignore_what_earlier_kernels_left_in_lds(hip, d, dv, sq, s
             np.testing.assert_allclose(a, w, rtol=2e-2, atol=1e-2 * max(1.0, np.abs(w).max()), err_msg=f"{name} {mode}")
 
 
+# batch, queries, keys, heads, key heads, head dim, causal, dtype, workgroups that share a row tile's keys (0: one)
+DIVIDED_KEYS = [
+    (1, 1, 1, 1, 1, 64, True, 1, 0), (2, 1, 31, 4, 2, 128, True, 2, 0), (1, 40, 40, 4, 2, 32, True, 2, 0),  # too few keys
+    (3, 4, 517, 8, 2, 64, True, 2, 0), (1, 33, 300, 2, 1, 128, True, 1, 0), (2, 7, 260, 6, 1, 96, False, 1, 0),
+    (1, 100, 611, 3, 3, 64, True, 1, 0),
+    (1, 1, 1000, 4, 4, 128, True, 1, 4), (1, 1, 4099, 16, 1, 40, False, 2, 11),  # one row tile
+    (1, 1000, 1000, 4, 1, 64, True, 1, 4), (1, 333, 2100, 4, 1, 128, True, 2, 6), (1, 200, 2099, 8, 2, 64, False, 1, 6),
+    # (batch, key head)s in whole eights, so in their XCDs' order
+    (2, 70, 1500, 8, 4, 64, True, 1, 4), (1, 45, 1300, 16, 8, 128, False, 2, 4), (1, 97, 1031, 8, 8, 96, True, 1, 3),
+    (4, 100, 700, 8, 8, 64, True, 2, 2)]
+
+
 @pytest.mark.parametrize("workspace", [True, False])
-@pytest.mark.parametrize("case", [
-    (1, 1, 1, 1, 1, 64, True, 1), (2, 1, 31, 4, 2, 128, True, 2), (1, 1, 1000, 4, 4, 128, True, 1),
-    (3, 4, 517, 8, 2, 64, True, 2), (1, 33, 300, 2, 1, 128, True, 1), (2, 7, 260, 6, 1, 96, False, 1),
-    (1, 40, 40, 4, 2, 32, True, 2), (1, 100, 611, 3, 3, 64, True, 1), (1, 1, 4099, 16, 1, 40, False, 2)])
+@pytest.mark.parametrize("case", DIVIDED_KEYS)
 def test_forward_with_keys_divided_over_waves(hip, case, workspace):
     """Few query rows: O and LSE against float64 for one and several row tiles, tiles that hold rows of several
-    heads of a group, key counts around the 32-key tiles and the waves' and workgroups' shares, padded head dims;
-    with a workspace (keys split over workgroups) and without."""
-    b, sq, sk, n, nkv, d, causal, dt = case
+    heads of a group, key counts around the 32-key tiles and the waves' and workgroups' shares, splits wholly past a
+    row tile's causal limit, padded head dims; with a workspace (keys split over workgroups) and without. The first
+    three have too few keys and stay with the general kernel."""
+    b, sq, sk, n, nkv, d, causal, dt, splits = case
     rng = np.random.default_rng(sk + d)
     np_t = np.float16
     bits = D.bf16_bits if dt == 1 else lambda x: x.astype(np_t).view(np.uint16)
@@ -333,8 +343,8 @@ def test_forward_with_keys_divided_over_waves(hip, case, workspace):
     desc = attn_desc(b, sq, sk, n, nkv, d, causal, 1.0 / math.sqrt(d), dtype=dt)
     size = C.c_size_t()
     nv.call("nhip_flash_fwd_workspace", C.byref(desc), C.byref(size))
-    if sk > 4000:
-        assert size.value > 0  # 1 head of 4099 keys is split over workgroups
+    rows = n // nkv * sq
+    assert size.value == splits * b * nkv * -(-rows // 32) * min(32, rows) * (4 * d + 8)
     dq, dk, dv, o, lse = Dev(q), Dev(k), Dev(v), Dev(nbytes=q.nbytes), Dev(nbytes=b * n * sq * 4)
     ws = Dev(nbytes=size.value)
     nv.call("nhip_flash_fwd_ws", C.byref(desc), dq.ptr, dk.ptr, dv.ptr, o.ptr, lse.ptr, ws.ptr if workspace else None)
