@@ -1296,6 +1296,8 @@ class LoopKernel:
             T = min(self.ROW_MAX_THREADS, max(64, -(-per // 64) * 64))
             rows_per_block = 1
         J = -(-chunks // T)
+        if sums and (J * V > self.SUM_COLUMNS or J * V * len(sums) > self.SUM_REGISTERS):
+            raise Unfusable(next(iter(sums)), "column sums of a row too wide for a thread's registers")
         exact = C % (T * V) == 0
         # column indices in 32 bits when the row allows (they stay live across the row's passes)
         cty, csuf = ("int", "") if C < (1 << 31) else ("int64_t", "LL")
@@ -1410,10 +1412,19 @@ class LoopKernel:
     # Row kernels that sum columns: 512 threads (several rows at once) a workgroup, at most SUM_BLOCKS workgroups of at
     # least SUM_ROWS rows a row group. Each stores its sums and a second kernel adds them: atomic adds by every
     # workgroup to one [C] vector cost 0.19 us an add and address, one after another (a [16384, 2048] norm backward
-    # 107 us with 256 workgroups, 146 with 512, 238 with 1024; 53 with stored sums).
+    # 107 us with 256 workgroups, 146 with 512, 238 with 1024; 53 with stored sums). Few rows: fewer rows a group rather
+    # than under SUM_FEW workgroups.
+    # A thread holds a sum for each of its columns beside the row's own values, so rows are at most SUM_COLUMNS columns a
+    # thread wide (16384, 8 at a time) and their sums at most SUM_REGISTERS together: wider ones spill. [R, C] norm
+    # backward in us with the sums here and in reductions of their own: [256, 16384] 24, 27; [4096, 16384] 114, 260; scale
+    # and shift, [4096, 12288] (48 registers) 124, 297. Past it: [256, 24576] 45, 33; scale and shift [256, 16384] 58, 44;
+    # a vocabulary head's bias, 8192 rows of 32000 1783, 1532, of 50304 (394 VGPRs spilled) 5059, 2293.
     SUM_THREADS = 512
     SUM_BLOCKS = 512
+    SUM_FEW = 64
     SUM_ROWS = 4
+    SUM_COLUMNS = 32
+    SUM_REGISTERS = 48
 
     def _row_sums(self, body, pro, stores, T, J, V, R, C, sums):
         """The row kernel ``body`` over many rows a workgroup, with each thread's column sums kept in registers: the
@@ -1421,7 +1432,7 @@ class LoopKernel:
         value, which ``<name>_sum<k>`` adds up."""
         groups = max(1, self.SUM_THREADS // T)
         threads = groups * T
-        blocks = max(1, min(self.SUM_BLOCKS, -(-R // (groups * self.SUM_ROWS))))
+        blocks = min(self.SUM_BLOCKS, max(-(-R // (groups * self.SUM_ROWS)), min(self.SUM_FEW, -(-R // groups))))
         self.grid, self.block, self.lds = (blocks, 1, 1), (threads, 1, 1), 0
         accs = [(k, j, l) for k in range(len(sums)) for j in range(J) for l in range(V)]
         src = [f'extern "C" __global__ __launch_bounds__({threads}) void {self.name}({self._params()}) {{',

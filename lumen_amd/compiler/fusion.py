@@ -599,7 +599,7 @@ def column_sums(graph, steps):
 
 def _row_kernel_ok(graph, st):
     """Whether a row kernel that sums columns can be generated for ``st`` (a row of one column has no column for the
-    generator to tell from the row)."""
+    generator to tell from the row, and a wide one more sums than a thread has registers)."""
     from lumen_amd.compiler import codegen
 
     def views(values):
@@ -613,10 +613,12 @@ def _row_kernel_ok(graph, st):
 
 
 def colsum_bytes(space):
-    """Scratch bytes of one value's column sums in a row kernel: a float32 row a workgroup."""
-    from lumen_amd.compiler.codegen import LoopKernel
+    """Scratch bytes of one value's column sums in a row kernel: a float32 row a workgroup (LoopKernel._row_sums's
+    count at one row group a workgroup, its most)."""
+    from lumen_amd.compiler.codegen import LoopKernel as K
 
-    return min(LoopKernel.SUM_BLOCKS, -(-space[0] // LoopKernel.SUM_ROWS)) * space[1] * 4
+    blocks = max(-(-space[0] // K.SUM_ROWS), min(K.SUM_FEW, space[0]))
+    return min(K.SUM_BLOCKS, blocks) * space[1] * 4
 
 
 COLSUM_MIN_ROWS = 256  # fewer rows: not worth a kernel that adds the workgroups' sums

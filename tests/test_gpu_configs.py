@@ -561,7 +561,8 @@ def test_gelu_gradient_closed_form_matches_float64():
     assert np.all(np.isnan(got[n + 4:])), got[n + 4:]
 
 
-@pytest.mark.parametrize("rows,cols", [(256, 64), (257, 72), (1000, 100), (700, 520), (3001, 2048), (300, 8192), (259, 1111)])
+@pytest.mark.parametrize("rows,cols", [(256, 64), (257, 72), (1000, 100), (700, 520), (3001, 2048), (300, 8192), (259, 1111), (1100, 1024),
+                                       (260, 12289), (300, 16384)])
 def test_norm_backward_row_kernel_sums_its_weight_gradient(hip, rows, cols):
     """RMS norm forward and backward in float32 as one row kernel with the weight's gradient summed over the rows it
     takes (one and several rows at a time, ragged row counts and row widths), against float64: the sum within the
@@ -576,7 +577,7 @@ def test_norm_backward_row_kernel_sums_its_weight_gradient(hip, rows, cols):
 
     f = L.compile(train, device="hip")
     args = [L.from_numpy(a).to("hip") for a in (x, w, dy)]
-    for _ in range(2):  # the second call adds into sums the first one left
+    for _ in range(2):  # the second call depends on nothing that the first left in its scratch or outputs
         y, dx, dw = (L.to_numpy(t) for t in f(*args))
     assert any(st.colsums for st in f.plan.steps)
     x6, w6, g6 = x.astype(np.float64), w.astype(np.float64), dy.astype(np.float64)
@@ -588,6 +589,35 @@ def test_norm_backward_row_kernel_sums_its_weight_gradient(hip, rows, cols):
     assert np.abs(dx - want).max() <= 1e-5 * np.abs(want).max()
     bound = (rows + 8) * 2.0**-24 * np.abs(terms).sum(0)
     assert np.all(np.abs(dw - terms.sum(0)) <= bound)
+
+
+@pytest.mark.parametrize("rows,cols,sums", [(256, 2, 2), (300, 72, 2), (1000, 1024, 2), (259, 5003, 2), (513, 12288, 2),
+                                            (270, 16384, 1), (300, 24576, 0)])
+def test_scale_and_shift_gradients_sum_in_one_row_kernel(hip, rows, cols, sums):
+    """A layer norm with scale and shift, bfloat16 operands: both gradients summed in the row kernel (each its part of
+    the scratch, the row groups' sums one after the other through the same LDS), one of them or none where a thread
+    has no registers for them; against float64 within the rounding of the float32 sums and of bfloat16."""
+    rng = np.random.default_rng(rows + cols)
+    x, dy, w, b = (D.bf16_to_f32(D.bf16_bits(rng.standard_normal(s).astype(np.float32)))
+                   for s in ((rows, cols), (rows, cols), (cols,), (cols,)))
+
+    def train(x, w, b, dy):
+        y, pull = L.vjp(lambda x, w, b: F.layer_norm(x.float(), x.shape[-1]) * w.float() + b.float(), x, w, b)
+        return [y, *pull(dy)]
+
+    f = L.compile(train, device="hip")
+    args = [L.tensor(a, "bfloat16").to(device="hip") for a in (x, w, b)] + [L.tensor(dy, "float32").to(device="hip")]
+    for _ in range(2):
+        _, _, dw, db = f(*args)
+    assert sum(len(st.colsums) for st in f.plan.steps) == sums
+    dw, db = (D.bf16_to_f32(t.raw()) for t in (dw, db))
+    x6, g6 = x.astype(np.float64), dy.astype(np.float64)
+    mid = x6 - x6.mean(1, keepdims=True)
+    norm = mid / np.sqrt((mid * mid).mean(1, keepdims=True) + 1e-5)
+    for got, terms in ((dw, g6 * norm), (db, g6)):
+        want = terms.sum(0)
+        bound = 2.0**-8 * np.abs(want) + (rows + 16) * 2.0**-23 * np.abs(terms).sum(0)
+        assert np.all(np.abs(got - want) <= bound)
 
 
 @pytest.mark.parametrize("m,k,n,dt", [(1, 33, 5, "float32"), (3, 64, 70, "float32"), (250, 97, 129, "float32"),

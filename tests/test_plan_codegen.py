@@ -657,3 +657,33 @@ def test_a_returned_attention_output_is_no_in_place_update(monkeypatch):
 def test_float32_folds_take_their_consumer_at_every_size(m, n, k):
     p = _plan(lambda x, w: F.relu(F.matmul(x, w, "float32", "float32")), ((m, k), "float32"), ((k, n), "float32"))
     assert [st.kind for st in p.steps] == ["dot"] and p.steps[0].epi_layout[1][0] == "fold"
+
+
+def test_column_sums_stay_apart_where_a_thread_has_no_registers_for_them():
+    """The weight gradients of norms over wide rows, and of a vocabulary head's bias: in the row kernel while a thread's
+    columns fit its registers (32, 48 sums in all), in reductions of their own past that."""
+    def norm(x, w, dy):
+        y, pull = L.vjp(lambda x, w: F.rms_norm(x.float(), x.size(-1), w.float()).bfloat16(), x, w)
+        return [y, *pull(dy)]
+
+    def scaled(x, w, b, dy):
+        y, pull = L.vjp(lambda x, w, b: (F.layer_norm(x.float(), x.shape[-1]) * w.float() + b.float()).bfloat16(), x, w, b)
+        return [y, *pull(dy)]
+
+    def head(h, w, b, t):
+        def loss(h, w, b):
+            return F.mean(F.cross_entropy(F.matmul(h, w.t(), "float32", "float32") + b.float(), t))
+
+        return L.value_and_grad(loss, (0, 1, 2))(h, w, b)[1]
+
+    def sums(p):
+        return [len(st.colsums) for st in p.steps if st.colsums], sum(st.kind == "reduce" for st in p.steps)
+
+    bf = "bfloat16"
+    for cols, want in ((16384, ([1], 0)), (16392, ([], 1)), (24576, ([], 1))):
+        assert sums(_plan(norm, ((512, cols), bf), ((cols,), bf), ((512, cols), bf))) == want
+    for cols, want in ((12288, ([2], 0)), (16384, ([1], 1)), (24576, ([], 2))):
+        p = _plan(scaled, ((512, cols), bf), ((cols,), bf), ((cols,), bf), ((512, cols), bf))
+        assert sums(p) == want
+    for vocab, want in ((16384, ([1], 0)), (32000, ([], 1)), (128256, ([], 1))):
+        assert sums(_plan(head, ((512, 64), bf), ((vocab, 64), bf), ((vocab,), bf), ((512,), "int64"))) == want
