@@ -181,7 +181,7 @@ int nhip_flash_fwd_ws(const nhip_attn_desc *desc, const void *q, const void *k, 
                       void *workspace);
 int nhip_flash_fwd_workspace(const nhip_attn_desc *desc, size_t *bytes);
 /* Number of forward tile configs nhip_attn_desc.config accepts (0: 128 queries a workgroup; 1: 256; 2: 64; by
- * default 0, or 2 at head dims to 64 with at most 64 queries) for autotuning and forced configs (the CUDA attention `Config`,
+ * default 0, or 2 at head dims to 64 with at most 64 queries of many heads) for autotuning and forced configs (the CUDA attention `Config`,
  * lumen/codegen/attention/cuda/mod.rs:312-420). */
 int nhip_attn_config_count(int *count);
 /* FlashAttention-2 backward (kernel.py:107-256): delta = rowsum(dO * O) (float32 [B, N, Sq]), then dK, dV

@@ -1239,10 +1239,10 @@ int launch_fwd(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *
         // head dim 256: 4 waves, one workgroup a CU (its K/V tiles fill 128 KiB of LDS), whatever the config
         return launch_fwd_nw<D, F16, CAUSAL, 4>(s, p, d);
     } else {
-        // by default 128 queries a workgroup, or 64 at head dim 64 where there are no more: waves without a query
-        // hold registers that others could use ([32, 1, 32 / 8, 64] over 1 key 8.9 us, 6.6; over 65 11.6, 7.8; 64 queries
-        // over 256 keys 18.9, 16.9)
-        switch (d->config >= 0 ? d->config : D == 64 && d->sq <= 64 ? 2 : 0) {
+        // by default 128 queries a workgroup, or 64 at head dim 64 where there are no more and the workgroups are more
+        // than the CUs hold, three each: waves without a query hold registers that others could use ([32, 1, 32 / 8, 64]
+        // over 1 key 8.9 us, 6.6; over 65 11.6, 7.8; 64 queries over 256 keys 18.9, 16.9; but [32, 1, 16, 64] 5.8, 6.2)
+        switch (d->config >= 0 ? d->config : D == 64 && d->sq <= 64 && d->heads * d->batch > 768 ? 2 : 0) {
             case 1: return launch_fwd_nw<D, F16, CAUSAL, 8>(s, p, d);
             case 2: return launch_fwd_nw<D, F16, CAUSAL, 2>(s, p, d);
             default: return launch_fwd_nw<D, F16, CAUSAL, 4>(s, p, d);

@@ -365,8 +365,9 @@ def test_forward_with_keys_divided_over_waves(hip, case, workspace):
 
 @pytest.mark.parametrize("sq,sk,d,causal", [(1, 1, 64, True), (40, 65, 64, True), (64, 64, 48, False), (65, 65, 64, True)])
 def test_default_forward_tile_gives_the_configs_bits(hip, sq, sk, d, causal):
-    """The workgroup size the forward picks by itself (64 queries up to 64 of them, else 128) changes no bit."""
-    b, n = 64, 8  # enough heads that the keys are not divided
+    """The workgroup size the forward picks by itself (64 queries up to 64 of them over many heads, else 128) changes no
+    bit."""
+    b, n = 100, 8  # enough heads for 64-query workgroups, and that the keys are not divided
     rng = np.random.default_rng(sq)
     q, k, v = (D.bf16_bits(rng.standard_normal(s).astype(np.float32)) for s in ((b, sq, n, d), (b, sk, n, d), (b, sk, n, d)))
     desc = attn_desc(b, sq, sk, n, n, d, causal, 1.0 / math.sqrt(d))
