@@ -602,11 +602,11 @@ def test_scale_and_shift_gradients_sum_in_one_row_kernel(hip, rows, cols, sums):
                    for s in ((rows, cols), (rows, cols), (cols,), (cols,)))
 
     def train(x, w, b, dy):
-        y, pull = L.vjp(lambda x, w, b: F.layer_norm(x.float(), x.shape[-1]) * w.float() + b.float(), x, w, b)
+        y, pull = L.vjp(lambda x, w, b: (F.layer_norm(x.float(), x.shape[-1]) * w.float() + b.float()).bfloat16(), x, w, b)
         return [y, *pull(dy)]
 
     f = L.compile(train, device="hip")
-    args = [L.tensor(a, "bfloat16").to(device="hip") for a in (x, w, b)] + [L.tensor(dy, "float32").to(device="hip")]
+    args = [L.tensor(a, "bfloat16").to(device="hip") for a in (x, w, b, dy)]
     for _ in range(2):
         _, _, dw, db = f(*args)
     assert sum(len(st.colsums) for st in f.plan.steps) == sums
