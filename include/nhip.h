@@ -180,9 +180,12 @@ int nhip_flash_fwd(const nhip_attn_desc *desc, const void *q, const void *k, con
 int nhip_flash_fwd_ws(const nhip_attn_desc *desc, const void *q, const void *k, const void *v, void *o, float *lse,
                       void *workspace);
 int nhip_flash_fwd_workspace(const nhip_attn_desc *desc, size_t *bytes);
+/* Whether that is so for `desc` (with or without a workspace): its result then differs from the tile configs', which all
+ * give the same bits, by the order of its float32 sums. */
+int nhip_flash_fwd_divides_keys(const nhip_attn_desc *desc, int *divides);
 /* Number of forward tile configs nhip_attn_desc.config accepts (0: 128 queries a workgroup; 1: 256; 2: 64; by
- * default 0, or 2 at head dims to 64 with at most 64 queries of many heads) for autotuning and forced configs (the CUDA attention `Config`,
- * lumen/codegen/attention/cuda/mod.rs:312-420). */
+ * default 0, or 2 at head dims to 64 with at most 64 queries of many heads, or divided keys) for autotuning and forced
+ * configs (the CUDA attention `Config`, lumen/codegen/attention/cuda/mod.rs:312-420). */
 int nhip_attn_config_count(int *count);
 /* FlashAttention-2 backward (kernel.py:107-256): delta = rowsum(dO * O) (float32 [B, N, Sq]), then dK, dV
  * per key block, and dQ by desc->deterministic's mode: from the dS tiles the dK/dV kernel stored (1), per query

@@ -73,16 +73,21 @@ static nhipk::SplitParams split_params(const nhip_attn_desc *d, int64_t *cost) {
     return sp;
 }
 
-// Where the longest workgroup of flash_fwd_kernel (every key, two workgroups a CU at once) would take longer. Measured
-// (us, flash_fwd_kernel and this; batch, queries, keys, heads / key heads, head dim): 16, 1, 4096, 16 / 16, 128:
-// 151, 97 (5.5 TB/s); 1, 1, 4096, 16 / 16, 128: 109, 20; 3, 1, 27958, 16 / 16, 128: 923, 126; 21, 1, 963, 32 / 8,
-// 64: 38, 15; 1, 1000, 1000, 4 / 1, 64: 22, 15; 1, 6180, 6180, 4 / 1, 64: 142, 110. Not: 4, 512, 512, 8 / 8, 128: 18,
-// 23; 2, 1777, 1777, 16 / 4, 64: 44, 54; 2, 58, 58, 16 / 16, 64: 5.4, 6.5.
+// Where flash_fwd_kernel would clearly take longer: its longest workgroup, every key, or where they are more than the
+// chip holds (two a CU, three at head dim 64) their total. Dividing the keys shares a tile of them between fewer
+// queries, so it has to be the faster by a third, less a small constant that few keys gain. Of 900 measured shapes
+// where a division's cost is below that time, this keeps 832, one of which the division slows by more than 5% (10%); of
+// the others, 36 (to 1.8 times). us of flash_fwd_kernel and this (batch, queries, keys, heads / key heads, head dim): 16, 1,
+// 4096, 16 / 16, 128: 151, 97 (5.5 TB/s); 1, 1, 4096, 16 / 16, 128: 109, 20; 3, 1, 27958, 16 / 16, 128: 923, 126; 21, 1,
+// 963, 32 / 8, 64: 38, 15; 1, 1000, 1000, 4 / 1, 64: 22, 15. Not: 2, 8310, 8310, 4 / 1, 40: 165, 301; 26, 599, 1661,
+// 4 / 1, 40: 51, 77; 2, 317, 21981, 32 / 32, 96: 532, 730; 4, 512, 512, 8 / 8, 128: 18, 23.
 bool split_keys(const nhip_attn_desc *d) {
     if (d->config >= 0 || kernel_dim(d) > 128 || d->sk == 0) return false;
     int64_t cost;
     split_params(d, &cost);
-    return cost < 4 * ((d->sk + 63) / 64) * (((d->sq + 127) / 128 * d->heads * d->batch + 511) / 512);
+    const int64_t slots = kernel_dim(d) == 64 ? 768 : 512;
+    const int64_t whole = 4 * ((d->sk + 63) / 64) * std::max(slots, (d->sq + 127) / 128 * d->heads * d->batch) / slots;
+    return cost < whole && 3 * cost < 2 * whole + 40;
 }
 
 static size_t fwd_workspace_bytes(const nhip_attn_desc *d) {
@@ -147,6 +152,13 @@ int nhip_flash_fwd_workspace(const nhip_attn_desc *desc, size_t *bytes) {
     *bytes = 0;
     if (check_attn(desc, "flash attention", 256)) return 1;
     *bytes = fwd_workspace_bytes(desc);
+    return 0;
+}
+
+int nhip_flash_fwd_divides_keys(const nhip_attn_desc *desc, int *divides) {
+    *divides = 0;
+    if (check_attn(desc, "flash attention", 256)) return 1;
+    *divides = split_keys(desc);
     return 0;
 }
 

@@ -131,6 +131,7 @@ SIGNATURES = {
     "nhip_flash_fwd": ([C.POINTER(AttnDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "nhip_flash_fwd_ws": ([C.POINTER(AttnDesc)] + [C.c_void_p] * 6, C.c_int),
     "nhip_flash_fwd_workspace": ([C.POINTER(AttnDesc), C.POINTER(C.c_size_t)], C.c_int),
+    "nhip_flash_fwd_divides_keys": ([C.POINTER(AttnDesc), C.POINTER(C.c_int)], C.c_int),
     "nhip_flash_bwd": (
         [C.POINTER(AttnDesc)] + [C.c_void_p] * 10,
         C.c_int,

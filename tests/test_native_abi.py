@@ -67,3 +67,20 @@ def test_gemm_kernel_says_what_nhip_gemm_would_run():
     assert kernel(4096, 4096, 4096, bf16)[0] == native.NHIP_GEMM_TILED
     assert kernel(300, 5003, 511, bf16)[0] == native.NHIP_GEMM_ANY
     assert kernel(300, 500, 0, bf16)[0] == native.NHIP_GEMM_EXACT
+
+
+def test_forwards_divide_their_keys_where_the_general_kernel_is_slower():
+    """Few query rows over many keys, and not the shapes measured slower that way (many row tiles), nor a forced tile."""
+    def divides(b, sq, sk, n, nkv, d, config=-1):
+        a = native.AttnDesc(batch=b, heads=n, kv_heads=nkv, sq=sq, sk=sk, head_dim=d, dtype=1, causal=1, scale=1.0, config=config)
+        out = C.c_int()
+        native.call("nhip_flash_fwd_divides_keys", C.byref(a), C.byref(out))
+        return bool(out.value)
+
+    for shape in [(16, 1, 4096, 16, 16, 128), (1, 1, 4096, 16, 16, 128), (3, 1, 27958, 16, 16, 128), (21, 1, 963, 32, 8, 64),
+                  (1, 1000, 1000, 4, 1, 64), (1, 333, 2100, 4, 1, 128), (3, 4, 517, 8, 2, 64), (16, 1, 1200, 32, 32, 40)]:
+        assert divides(*shape) and not divides(*shape, config=0), shape
+    for shape in [(2, 8310, 8310, 4, 1, 40), (26, 599, 1661, 4, 1, 40), (2, 317, 21981, 32, 32, 96), (1, 1156, 1895, 16, 16, 64),
+                  (12, 60, 3355, 32, 32, 64), (2, 1194, 23358, 32, 8, 64), (4, 512, 512, 8, 8, 128), (2, 1777, 1777, 16, 4, 64),
+                  (2, 58, 58, 16, 16, 64), (1, 1, 1, 1, 1, 64), (1, 1, 4096, 16, 16, 256)]:
+        assert not divides(*shape), shape
