@@ -11,6 +11,7 @@ then queues every step on the device's stream with no host work per step but the
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 import math
 import struct
 from dataclasses import dataclass, replace
@@ -561,8 +562,11 @@ class Plan:
 
     def _fuse_epilogues(self):
         """Merges each loop step that is the elementwise consumer of a dot's [m, n] result into the dot's step
-        (``st.epi``); returns whether any was merged. The loop's other inputs must exist before the dot runs;
-        the dot's result is still stored when other steps or the graph's outputs read it."""
+        (``st.epi``); returns whether any was merged. The dot runs in its place, or (without a memory limit: values may
+        live longer) in the loop's where the loop reads values made between the two and nothing else there reads the
+        dot's result: an order that puts a dot first then costs no pass (the product and GELU backward of a [4096, 2048,
+        8192] MLP run as one kernel in 168 us, the product alone in 139). The dot's result is still stored when other
+        steps or the graph's outputs read it."""
         from lumen_amd.graph.ir import ELEMENTWISE
 
         g = self.graph
@@ -574,8 +578,9 @@ class Plan:
             for u in st.inputs:
                 users.setdefault(u, []).append(si)
         outputs = set(g.outputs)
-        merged = set()
-        for si, st in enumerate(self.steps):
+        merged, at = set(), {}  # steps that leave their place; dots that take a loop's
+        dots = {st.nodes[0].output for st in self.steps if st.kind == "dot"}
+        for moves, (si, st) in itertools.product((False, True), enumerate(self.steps)):
             if st.kind != "dot" or getattr(st, "epi", None) is not None:
                 continue
             dv = st.nodes[0].output
@@ -583,7 +588,8 @@ class Plan:
             if lay is None:
                 continue
             shape = g.types[dv].shape
-            for li in users.get(dv, []):
+            # loops that read no other dot's result first: that dot may move to one that does
+            for li in sorted(users.get(dv, []), key=lambda li: any(u in dots and u != dv for u in self.steps[li].inputs)):
                 lt = self.steps[li]
                 if li in merged or lt.kind != "loop" or li <= si:
                     continue
@@ -592,8 +598,9 @@ class Plan:
                 readers = [n for n in lt.nodes if dv in n.inputs]
                 if any(n.prim not in ELEMENTWISE or g.types[n.output].shape != shape for n in readers):
                     continue
-                if any(u != dv and pos.get(u, -1) >= si for u in lt.inputs):
-                    continue  # an operand the loop reads is made after the dot
+                late = any(u != dv and pos.get(u, -1) >= si for u in lt.inputs)  # made after the dot
+                if late and (not moves or config.compiler.memory_limit or any(x < li for x in users[dv])):
+                    continue
                 keep = dv in outputs or any(x != li for x in users.get(dv, []))
                 outs = ([dv] if keep else []) + list(lt.outputs)
                 try:  # past its first readers the loop may read the result at other elements (exp(y) + exp(y).t())
@@ -607,8 +614,12 @@ class Plan:
                 st.inputs = list(st.inputs) + [u for u in lt.inputs if u != dv and u not in st.inputs]
                 st.nodes = list(st.nodes) + list(lt.nodes)
                 merged.add(li)
+                if late:
+                    at[li] = st
+                    merged.add(si)
+                    pos[dv] = li
                 break
-        self.steps = [st for i, st in enumerate(self.steps) if i not in merged]
+        self.steps = [at.get(i, st) for i, st in enumerate(self.steps) if i not in merged or i in at]
         return bool(merged) | self._fuse_column_sums()
 
     def _epilogue_kernel(self, st, loop, layout, store_dot, outputs, colsum=None, variant=0):

@@ -6,6 +6,8 @@ import pytest
 import lumen_amd as L
 import lumen_amd.functional as F
 from lumen_amd import dtypes as D
+from lumen_amd import workloads as W
+from lumen_amd.compiler.plan import Plan
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -664,3 +666,29 @@ def test_small_update_in_place_reads_each_weight_once(hip):
         for i in range(k):
             fold += x[:, i, None] * y[i]
         np.testing.assert_allclose(L.to_numpy(dev[0]), w - np.float32(0.5) * fold, rtol=0, atol=1e-6)
+
+
+def test_dots_that_move_to_their_consumer_keep_their_bits(hip, monkeypatch):
+    """A block in training in the order that puts its output gradient's product first: the product runs where the GELU's
+    backward does, with that in its store, and all outputs keep the bits of the plan without fused stores."""
+    monkeypatch.setattr(Plan, "EPI_MIN_TILES", 1)
+    cfg = W.TransformerConfig(vocab=8, dim=64, heads=1, ffn=264, seq=300, batch=1, layers=1)
+    model = W.build(cfg, lr=1.0)[0]
+    W.load(model, W.init_weights(model))
+    rng = np.random.default_rng(9)
+    x, dy = (L.tensor(rng.standard_normal((300, 64)).astype(np.float32), "bfloat16").to(device="hip") for _ in range(2))
+
+    def train(block, x, dy):
+        y = block(x, 1, 1)
+        y.backward(dy)
+        return [y, x.grad, *(p.grad for p in block.parameters())]
+
+    outs = []
+    for fuse in (True, False):
+        with L.config.compiler.patch(schedules=False, horizontal_fusion=False, epilogue_fusion=fuse, autotune=False):
+            f = L.compile(train, device="hip")
+            outs.append([t.raw().copy() for t in f(model.layers[0], x, dy)])
+        stores = [st.epi.label() for st in f.plan.steps if getattr(st, "epi", None) is not None]
+        assert len(stores) >= 2 * fuse
+    for got, want in zip(*outs):
+        np.testing.assert_array_equal(got, want)

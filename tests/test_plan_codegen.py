@@ -687,3 +687,33 @@ def test_column_sums_stay_apart_where_a_thread_has_no_registers_for_them():
         assert sums(p) == want
     for vocab, want in ((16384, ([1], 0)), (32000, ([], 1)), (128256, ([], 1))):
         assert sums(_plan(head, ((512, 64), bf), ((vocab, 64), bf), ((vocab,), bf), ((512,), "int64"))) == want
+
+
+def _block_train(block, x, dy, batch, heads):
+    y = block(x, batch, heads)
+    y.backward(dy)
+    return [y, x.grad, *(p.grad for p in block.parameters())]
+
+
+def test_a_dot_moves_to_its_consumer_past_what_that_reads():
+    """A dot ahead of a value that its elementwise consumer reads too (a block's output gradient times the second MLP
+    weight, ready before the forward that the GELU's backward needs) runs in the consumer's place with it in the store;
+    not where a step between the two reads the dot's result."""
+    cfg = W.TransformerConfig(vocab=8, dim=64, heads=1, ffn=4096, seq=4096, batch=1, layers=1)
+    block = W.build(cfg, lr=1.0)[0].layers[0]
+    x = L.empty([cfg.tokens, cfg.dim], "bfloat16", "meta")
+    for limit, fused in ((0, 2), (1 << 40, 1)):
+        with L.config.compiler.patch(schedules=False, memory_limit=limit):
+            p = Plan(trace(_block_train, (block, x, x, 1, 1)).graph, build_kernels=False)
+        assert sum(getattr(st, "epi", None) is not None for st in p.steps) == fused
+        made = set()
+        for st in p.steps:
+            assert all(u in made or u in p.graph.inputs for u in st.inputs)
+            made.update(st.outputs)
+
+    def read_between(x, w):
+        y = F.matmul(x, w.t(), "float32", "float32")
+        return y * F.sum(y, 0)
+
+    p = _plan(read_between, ((4096, 64), "bfloat16"), ((4096, 64), "bfloat16"))
+    assert [st.kind for st in p.steps if st.kind != "view"] == ["dot", "reduce", "loop"]
