@@ -198,7 +198,9 @@ __device__ __forceinline__ void load_tile_async(const uint16_t *src, int64_t rs,
 // when there are few query blocks. Two workgroups a CU hold the 64 KiB (D = 128) double-buffered tiles, so
 // each wave keeps 256 VGPRs at 4 waves a workgroup and 8 (one workgroup a CU at 8). At D = 64 a wave is held to 168
 // VGPRs, three waves a SIMD: left to itself a causal one takes 172 and two ([32, 1000, 16, 64] 164 us, 138 with three;
-// [8, 2048, 16, 64] 132, 117; [32, 512, 32 / 8, 64] 110, 92). Four spill 24 registers (173, 129, 108).
+// [8, 2048, 16, 64] 132, 117; [32, 512, 32 / 8, 64] 110, 92). Four spill 24 registers (173, 129, 108). Launches that two a
+// SIMD nearly hold at once keep the 172 (launch_fwd_nw; with two, three: [2, 1777, 16 / 4, 64], 448 workgroups, 36.5, 37.4 us;
+// [5, 1000, 16, 64], 640, 33.5, 34.0; [6, 1000, 16, 64], 768, 40.7, 34.6).
 template <int NW, int D = 128> struct FwdOccupancy {
     static constexpr int kBlocks = D > 128 ? 1 : NW >= 8 ? 1 : NW >= 4 ? (D > 64 ? 2 : 3) : 4;
 };
@@ -364,8 +366,8 @@ __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     if (h == 0 && p.lse) p.lse[(b * p.heads + n) * p.sq + qi] = l > 0.0f ? (m + __log2f(l)) * 0.6931471805599453f : -INFINITY;
 }
 
-template <int D, bool F16, bool CAUSAL, int NW = 4>
-__global__ __launch_bounds__(64 * NW, (FwdOccupancy<NW, D>::kBlocks)) void flash_fwd_kernel(AttnParams p) {
+template <int D, bool F16, bool CAUSAL, int NW = 4, int WAVES = FwdOccupancy<NW, D>::kBlocks>
+__global__ __launch_bounds__(64 * NW, WAVES) void flash_fwd_kernel(AttnParams p) {
     flash_fwd_body<D, F16, CAUSAL, NW>(p);
 }
 
@@ -1229,6 +1231,12 @@ inline int check_attn(const nhip_attn_desc *d, const char *what, int64_t max_hd 
 template <int D, bool F16, bool CAUSAL, int NW>
 int launch_fwd_nw(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *d) {
     dim3 grid(unsigned((d->sq + 32 * NW - 1) / (32 * NW) * d->heads * d->batch));
+    if constexpr (D == 64 && CAUSAL && NW == 4) {
+        if (grid.x <= 640) {
+            hipLaunchKernelGGL((nhipk::flash_fwd_kernel<D, F16, CAUSAL, NW, 2>), grid, dim3(64 * NW), 0, s, p);
+            return check(hipGetLastError(), "flash_fwd launch");
+        }
+    }
     hipLaunchKernelGGL((nhipk::flash_fwd_kernel<D, F16, CAUSAL, NW>), grid, dim3(64 * NW), 0, s, p);
     return check(hipGetLastError(), "flash_fwd launch");
 }
