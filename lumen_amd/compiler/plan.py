@@ -482,14 +482,10 @@ class Plan:
                 st.splits, split_cfg = (1, None) if getattr(st, "epi", None) is not None else self._split_count(st.nodes[0])
                 if split_cfg is not None:
                     st.config = split_cfg
-                st.split_choices, st.scratch = [st.splits], 0
-                if st.splits > 1 or split_cfg is not None:
+                st.scratch = 0
+                if st.splits > 1:
                     d, _ = self._gemm_desc(st.nodes[0])
-                    if config.compiler.autotune and not config.compiler.memory_limit:
-                        st.split_choices = self._split_choices(d, st.splits)
-                most = max(st.split_choices + [st.splits])
-                if most > 1:
-                    st.scratch = most * max(1, math.prod(d.batch[i] for i in range(d.nbatch))) * d.m * d.n * 4
+                    st.scratch = st.splits * max(1, math.prod(d.batch[i] for i in range(d.nbatch))) * d.m * d.n * 4
             if st.kind == "linear_cross_entropy":
                 st.scratch = self._lce_scratch(self._lce_desc(st.nodes[0]))
             if st.scratch:
@@ -1026,11 +1022,12 @@ class Plan:
 
     # ---- autotuning (lumen/autotune/mod.rs:20-150): bf16/f16 dots of at least 2^30 multiply-adds try every tile
     # config the kernel accepts, timed with HIP events on the step's own operands (their values do not change
-    # MFMA timing), before the first run; the fastest is kept per (shape, layout, dtype) for the process.
+    # MFMA timing), before the first run; the fastest is kept per (shape, layout, dtype) for the process. Only kernels
+    # that give the same bits are timed against each other, so that those of a plan do not depend on the timing:
+    # whether a dot's few rows or an attention's keys are divided, and into how many parts k, rules decide.
     AUTOTUNE_MACS = 1 << 30
     AUTOTUNE_MARGIN = 0.03
     _tuned: dict = {}
-    _tuned_splits: dict = {}  # dots: the split count timed with the config
 
     def _apply_forced(self):
         """Configs of ``lumen_amd.autotune.use`` blocks: every plain GEMM step (any size) and every flash
@@ -1106,9 +1103,9 @@ class Plan:
     ATTN_AUTOTUNE_FLOPS = 1 << 32  # flash forwards of fewer FLOPs keep the default tile
 
     def _autotune_attention(self, workspace_ptr, input_ptrs):
-        """Times the default and each forward tile config on a flash forward step's own operands (HIP events, 3 runs after a
+        """Times each forward tile config on a flash forward step's own operands (HIP events, 3 runs after a
         warm-up) and keeps the fastest (a later one must win by ``AUTOTUNE_MARGIN``); picks are shared by
-        steps of the same shape, layout and dtype."""
+        steps of the same shape, layout and dtype. A forward whose keys the library divides keeps that kernel."""
         from lumen_amd import native as nv
 
         n_cfg = C.c_int()
@@ -1121,6 +1118,10 @@ class Plan:
             if flops < self.ATTN_AUTOTUNE_FLOPS:
                 continue
             kind, desc, ops = attn_pass.lower(self, st)
+            divides = C.c_int()
+            nv.call("nhip_flash_fwd_divides_keys", C.byref(desc), C.byref(divides))
+            if divides.value:
+                continue
             key = ("attn", desc.batch, desc.heads, desc.kv_heads, desc.sq, desc.sk, desc.head_dim, desc.dtype,
                    desc.causal, desc.q_s, desc.k_s, desc.v_s, desc.o_s)
             if key not in Plan._tuned:
@@ -1128,15 +1129,13 @@ class Plan:
                 for loc in ops:
                     base = workspace_ptr if loc.base[0] == "ws" else input_ptrs[loc.base[1]]
                     ptrs.append(base + loc.offset * D.size_of(loc.dtype))
-                # the library's own choice first, which may divide the keys (through the step's workspace)
-                ptrs += [None] * (6 - len(ptrs))
-                best, best_ms = -1, float("inf")
-                for cfg in range(-1, n_cfg.value):
+                best, best_ms = 0, float("inf")
+                for cfg in range(n_cfg.value):
                     desc.config = cfg
-                    nv.call("nhip_flash_fwd_ws", C.byref(desc), *ptrs)  # warm-up
+                    nv.call("nhip_flash_fwd", C.byref(desc), *ptrs[:5])  # warm-up
                     ev0.record()
                     for _ in range(3):
-                        nv.call("nhip_flash_fwd_ws", C.byref(desc), *ptrs)
+                        nv.call("nhip_flash_fwd", C.byref(desc), *ptrs[:5])
                     ev1.record()
                     ms = ev0.elapsed_ms(ev1) / 3
                     if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
@@ -1153,18 +1152,15 @@ class Plan:
         for st in self.steps:
             if st.kind != "dot" or getattr(st, "epi", None) is not None or getattr(st, "forced", False):
                 continue
-            choices = getattr(st, "split_choices", [1])
-            if len(choices) == 1 and getattr(st, "splits", 1) > 1:
-                continue
             try:
                 d, ops = self._gemm_desc(st.nodes[0])
             except NotImplementedError:
                 continue
             z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
-            if d.a_dtype == nv.NHIP_F32 or d.m * d.n * d.k * z < self.AUTOTUNE_MACS:
+            if d.m * d.n * d.k * z < self.AUTOTUNE_MACS or _gemm_kernel(d, ops)[0] != nv.NHIP_GEMM_TILED:
                 continue
             key = (d.m, d.n, d.k, tuple(d.batch[i] for i in range(d.nbatch)), d.a_dtype, d.d_dtype,
-                   d.a_m == 1, d.a_k == 1, d.b_k == 1, d.b_n == 1, d.d_n == 1, tuple(choices))
+                   d.a_m == 1, d.a_k == 1, d.b_k == 1, d.b_n == 1, d.d_n == 1, st.splits)
             if key not in Plan._tuned:
                 ptrs = []
                 for loc in ops:
@@ -1172,49 +1168,59 @@ class Plan:
                     ptrs.append(base + loc.offset * D.size_of(loc.dtype))
                 scratch = self.scratch.get(id(st))
                 ptrs.append(workspace_ptr + scratch.offset * 4 if scratch is not None else None)
-                best, best_ms = (-1, 1), float("inf")
-                for splits in choices:
-                    for cfg in range(n_cfg.value) if splits == 1 else (self.STREAM128, self.STREAM8W):
-                        d.config, d.splits = cfg, splits
-                        try:  # warm-up; rejects configs the shape can't take
-                            nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
-                        except RuntimeError:
-                            continue
-                        ev0.record()
-                        for _ in range(3):
-                            nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
-                        ev1.record()
-                        ms = ev0.elapsed_ms(ev1) / 3
-                        # a later config must win by more than timing noise (3%), so near-ties pick the same
-                        # kernel run after run
-                        if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
-                            best, best_ms = (cfg, splits), ms
-                Plan._tuned_splits[key], Plan._tuned[key] = best[1], best[0]
-            st.config, st.splits = Plan._tuned[key], Plan._tuned_splits[key]
+                best, best_ms = -1, float("inf")
+                d.splits = st.splits
+                for cfg in range(n_cfg.value) if st.splits == 1 else (self.STREAM128, self.STREAM8W):
+                    d.config = cfg
+                    if _gemm_kernel(d, ops)[0] != nv.NHIP_GEMM_TILED:
+                        continue
+                    try:  # warm-up; rejects configs the shape can't take
+                        nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
+                    except RuntimeError:
+                        continue
+                    ev0.record()
+                    for _ in range(3):
+                        nv.call("nhip_gemm_splitk", C.byref(d), *ptrs)
+                    ev1.record()
+                    ms = ev0.elapsed_ms(ev1) / 3
+                    # a later config must win by more than timing noise (3%), so near-ties pick the same
+                    # kernel run after run
+                    if ms < best_ms * (1.0 - self.AUTOTUNE_MARGIN):
+                        best, best_ms = cfg, ms
+                Plan._tuned[key] = best
+            st.config = Plan._tuned[key]
 
-    # Split-k policy: a bf16/f16 dot whose 256 x 256 output tiles cannot fill the 256 CUs is cut along k (in
-    # powers of two, each part at least 1024 deep) until they do; its float32 partials live in the step's
-    # scratch (nhip_gemm_splitk).
+    # Split-k: a bf16/f16 dot whose 256 x 256 output tiles cannot fill the 256 CUs may be cut along k, in powers of
+    # two; its float32 partials live in the step's scratch (nhip_gemm_splitk). Dots too small to be timed are cut until
+    # they fill the chip, each part at least SPLIT_MIN_K deep; larger ones into the parts that _split_us makes the
+    # fastest, at least SPLIT_TIMED_MIN_K deep, with partials of at most SPLIT_BYTES (half that under a memory limit).
     SPLIT_MIN_K = 1024
     SPLIT_MAX = 8
     STREAM128 = 9  # kernels.hip's kStream128
     STREAM8W = 7  # kernels.hip's kStream8w
-    SPLIT_TUNED_MIN_K = 512
-    SPLIT_TUNED_BYTES = 256 << 20
+    SPLIT_TIMED_MIN_K = 512
+    SPLIT_BYTES = 64 << 20
 
-    def _split_choices(self, d, splits):
-        """The split counts the autotuner times for a dot the policy gives ``splits``: powers of two to SPLIT_MAX with
-        parts of at least SPLIT_TUNED_MIN_K and float32 partials within SPLIT_TUNED_BYTES. The policy only fills
-        the chip; whether that pays for writing and reading the partials depends on the shape: [8192, 2048] x [2048,
-        512] takes 28 us whole and 36 in two parts, [2048, 8192] x [8192, 512] 78 and 41 in eight."""
-        z = max(1, math.prod(d.batch[i] for i in range(d.nbatch)))
-        if d.m * d.n * d.k * z < self.AUTOTUNE_MACS or -(-d.m // 256) * -(-d.n // 256) * z >= 256:
-            return [splits]
-        s = [1]
-        while s[-1] < self.SPLIT_MAX and d.k % (128 * s[-1]) == 0 and d.k // (2 * s[-1]) >= self.SPLIT_TUNED_MIN_K \
-                and 8 * s[-1] * z * d.m * d.n <= self.SPLIT_TUNED_BYTES:
-            s.append(2 * s[-1])
-        return s
+    @staticmethod
+    def _split_us(d, z, splits):
+        """About the microseconds of a dot in ``splits`` parts by the best tile config: the rounds in which its 128 x 128
+        tiles (two a CU; at most one a CU takes 0.79 of a round), its 256 x 256 ones or, whole, its 64 x 64 ones (four a
+        CU, one a CU 0.59) fit on the chip, each k long, and the partials written and read. Fitted to 367 shapes of 2^30 to
+        2^38 multiply-adds in three layouts, each measured in 1, 2, 4 and 8 parts at its best config: the count this
+        gives is on average 0.6% slower than the fastest (at most 21%; filling the chip 2.7%, 39%; never dividing 44%).
+        [8192, 512] x [512, 2048] 28 us whole, 35 in two; [2048, 8192] x [8192, 512] 71, 54, 39, 37; [8192, 32000] x
+        [32000, 512] 477, 328, 282."""
+        def tiles(b):
+            return -(-d.m // b) * -(-d.n // b) * z
+
+        full, rest = divmod(tiles(128) * splits, 512)
+        small = full + (0 if rest == 0 else 0.79 if rest <= 256 else 1)
+        us = 6.2 + d.k / splits * min(0.0142 * small, 0.02355 * -(-tiles(256) * splits // 256))
+        if splits > 1:
+            return us + 4.2 + 8 * splits * z * d.m * d.n / 6.13e6
+        full, rest = divmod(tiles(64), 1024)
+        small = full + (0 if rest == 0 else 0.59 + 0.41 * max(0, rest - 256) / 768)
+        return min(us, 2.9 + 0.0154 * d.k * small)
 
     def _split_count(self, n):
         lhs, rhs, out = self.loc[n.inputs[0]], self.loc[n.inputs[1]], self.loc[n.output]
@@ -1230,6 +1236,13 @@ class Plan:
         tiles = -(-d.m // 256) * -(-d.n // 256) * z
         if tiles >= 256:
             return 1, None
+        if config.compiler.autotune and d.m * d.n * d.k * z >= self.AUTOTUNE_MACS \
+                and autotune.forced(autotune.HipGemmConfig) is None:
+            most = self.SPLIT_BYTES // (2 if config.compiler.memory_limit else 1)
+            counts = [s for s in (2, 4, 8) if d.k % (64 * s) == 0 and d.k // s >= self.SPLIT_TIMED_MIN_K
+                      and 4 * s * z * d.m * d.n <= most]
+            s = min([1] + counts, key=lambda s: self._split_us(d, z, s) * (1.03 if s > 1 else 1))
+            return s, (self.STREAM128 if s > 1 else -1)
         # the 128 x 128 kernel runs two workgroups a CU: split until its tiles fill 2 x 256 of them
         tiles = -(-d.m // 128) * -(-d.n // 128) * z
         s = 1

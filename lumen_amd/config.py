@@ -17,7 +17,9 @@ class CompilerFlags:
     merge_dots: bool = True           # one dot for dots sharing an operand (QKV)
     horizontal_fusion: bool = True    # merge small independent loop kernels into one launch
     epilogue_fusion: bool = True      # fuse elementwise consumers into GEMM stores
-    autotune: bool = True             # time GEMM tile candidates before a plan's first run
+    # time large GEMMs' tile configs and k loops and large attentions' workgroup sizes before a plan's first run: all
+    # give the same bits, so results do not depend on the timing
+    autotune: bool = True
     # attention backward without atomics: dQ by a kernel of its own (same bits every run); off, as in the
     # reference (graph_compiler/config/mod.rs:117), the dK/dV kernel adds dQ atomically
     deterministic: bool = True

@@ -5,8 +5,11 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import lumen_amd as L
+import lumen_amd.functional as F
 from lumen_amd import dtypes as D
 from lumen_amd import native as nv
+from lumen_amd.compiler.plan import Plan
 from tests.hiputil import Dev
 
 pytestmark = pytest.mark.gpu
@@ -47,6 +50,59 @@ def test_gemm_layouts(hip, at, bt, m, n, k, cfg):
     nv.call("nhip_gemm", C.byref(desc), da.ptr, db.ptr, dd.ptr)
     got = dd.get((m, n), np.float32)
     assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max() + 1e-4
+
+
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(264, 520, 512), (136, 72, 1024), (520, 264, 96), (72, 136, 200), (64, 264, 512)])
+def test_gemm_configs_agree_bit_for_bit(hip, at, bt, m, n, k):
+    """Every tile config gives the same bits, whole and in 2 or 4 parts of k, so that a plan's results do not depend on
+    which of them the autotuner times as the fastest. (Config 16, dots of few rows, sums in another order.)"""
+    rng = np.random.default_rng(m + n + k)
+    a, b = (D.bf16_bits(rng.standard_normal(s).astype(np.float32)) for s in ((m, k), (k, n)))
+    da, db, dd, dw = Dev(np.ascontiguousarray(a.T) if at else a), Dev(b if bt else np.ascontiguousarray(b.T)), \
+        Dev(nbytes=m * n * 4), Dev(nbytes=4 * m * n * 4)
+    desc = _desc(m, n, k, 1 if at else k, m if at else 1, n if bt else 1, 1 if bt else k)
+    for splits in (1, 2, 4):
+        if splits > 1 and k % (64 * splits):
+            continue
+        got = {}
+        for cfg in range(16):
+            desc.config, desc.splits = cfg, splits
+            if cfg >= 6 and k % (32 if cfg in (8, 11, 12, 13) else 64) or splits > 1 and cfg not in (7, 9):
+                continue
+            nv.call("nhip_gemm_splitk", C.byref(desc), da.ptr, db.ptr, dd.ptr, dw.ptr)
+            got[cfg] = dd.get((m, n), np.uint32)
+        first = next(iter(got.values()))
+        assert len(got) >= 2 and all(np.array_equal(x, first) for x in got.values()), \
+            (splits, [c for c, x in got.items() if not np.array_equal(x, first)])
+
+
+def test_only_kernels_of_the_same_bits_are_timed_against_each_other(hip, monkeypatch):
+    """The autotuner leaves alone a forward whose keys are divided, and never times the few-row kernel against the tiled
+    ones (both sum in another order): 64 rows of many columns run a tiled kernel by rule."""
+    timed = []
+    call = nv.call
+
+    def record(name, *args):
+        if name in ("nhip_gemm_splitk", "nhip_gemm", "nhip_flash_fwd", "nhip_flash_fwd_ws"):
+            timed.append((name, args[0]._obj.config))
+        return call(name, *args)
+
+    monkeypatch.setattr(nv, "call", record)
+    monkeypatch.setattr(Plan, "_tuned", {})
+
+    def fn(x, w, q, k, v):
+        return F.matmul(x, w.t(), "float32", "bfloat16"), F.flash_attention(q, k, v)
+
+    shapes = [(64, 2048), (32768, 2048), (2, 8, 64, 128), (2, 9000, 8, 128), (2, 9000, 8, 128)]
+    rng = np.random.default_rng(0)
+    block = rng.standard_normal(1 << 16).astype(np.float32)
+    f = L.compile(fn, device="hip")
+    f(*[L.tensor(np.resize(block, s), "bfloat16").to(device="hip") for s in shapes])
+    (flash,) = [i for i, st in enumerate(f.plan.steps) if st.kind == "flash_fwd"]
+    assert f.plan.cost(flash)[0] >= Plan.ATTN_AUTOTUNE_FLOPS  # large enough to be timed otherwise
+    assert {name for name, _ in timed} == {"nhip_gemm_splitk"} and {c for _, c in timed} == set(range(16))
+    assert [st.config for st in f.plan.steps if st.kind == "dot"][0] in range(16)
 
 
 def test_gemm_batched_bf16_output(hip):

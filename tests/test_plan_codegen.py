@@ -578,21 +578,20 @@ def test_norm_weight_gradient_sums_join_the_row_kernel():
     assert sum(len(st.colsums) for st in p.steps) >= 2
 
 
-def test_split_counts_are_timed_where_the_dot_is_large():
-    """A large dot whose 256 x 256 tiles do not fill the chip has scratch for every split count the autotuner times; a
-    small one, one that fills it, and a plan with a memory limit keep the policy's count."""
+def test_split_counts_follow_a_rule_and_need_only_their_own_scratch():
+    """Large dots whose 256 x 256 tiles do not fill the chip are cut into the parts that measured fastest, where one
+    count clearly did; the step has scratch for that count alone, within 64 MiB (half that under a memory limit)."""
     def dot(m, n, k):
         p = _plan(lambda x, w: F.matmul(x, w.t(), "float32", "bfloat16"), ((m, k), "bfloat16"), ((n, k), "bfloat16"))
         return next(st for st in p.steps if st.kind == "dot")
 
-    st = dot(8192, 512, 2048)
-    assert st.split_choices == [1, 2, 4] and st.scratch == 4 * 8192 * 512 * 4
-    assert dot(512, 2048, 8192).split_choices == [1, 2, 4, 8]
-    assert dot(8192, 8192, 512).split_choices == [1] and dot(8192, 8192, 512).scratch == 0
-    assert dot(256, 512, 1024).split_choices == [1] and dot(1000, 512, 8000).split_choices[0] == 1
+    for m, n, k, splits in [(8192, 512, 2048, 1), (4096, 2048, 2048, 1), (4096, 2048, 8192, 1), (2048, 8192, 4096, 1),
+                            (2048, 512, 8192, 8), (512, 2048, 8192, 8), (512, 512, 8192, 8), (8192, 512, 32000, 4),
+                            (3000, 1024, 32000, 4), (8192, 8192, 512, 1), (256, 512, 1024, 1), (1000, 512, 8000, 1)]:
+        st = dot(m, n, k)
+        assert st.splits == splits and st.scratch == (splits * m * n * 4 if splits > 1 else 0), (m, n, k, st.splits)
     with L.config.compiler.patch(memory_limit=1 << 40):
-        st = dot(512, 2048, 8192)
-        assert st.split_choices == [st.splits] == [8]
+        assert dot(512, 2048, 8192).splits == 8 and dot(8192, 512, 32000).splits == 2
 
 
 @pytest.mark.parametrize("m,k,n,dt", [(64, 64, 64, "float32"), (64, 64, 64, "bfloat16"), (16, 128, 16, "bfloat16"),
