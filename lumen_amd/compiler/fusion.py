@@ -550,6 +550,7 @@ def column_sums(graph, steps):
     kernels 4.69 ms and dots 55.3, and 77.6-78.2 in the stores, row kernels 4.30 and dots 56.1."""
     outputs = set(graph.outputs)
     pos, readers = {}, {}
+    at = {id(st): si for si, st in enumerate(steps)}  # list.index would compare steps field by field
     for si, st in enumerate(steps):
         for v in st.outputs:
             pos[v] = si
@@ -565,20 +566,21 @@ def column_sums(graph, steps):
                 or graph.types[red.output].dtype != "float32":
             continue
         space = (math.prod(x.shape[:-1]), x.shape[-1])
-        if space[0] < COLSUM_MIN_ROWS or u in outputs or u not in pos or readers.get(u) != [st]:
+        if space[0] < COLSUM_MIN_ROWS or u in outputs or u not in pos or len(readers[u]) != 1:
             continue
         made, moved = steps[pos[u]], []
-        reader = min((steps.index(r) for r in readers.get(red.output, [])), default=len(steps))
+        reader = min((at[id(r)] for r in readers.get(red.output, [])), default=len(steps))
         if made.kind == "row" and made.rows == space:
             row = made
         elif made.kind == "loop" and made.outputs == [u]:
             def takes(r):
-                ri = steps.index(r)
+                ri = at[id(r)]
+                if r.kind != "row" or r.rows != space or ri >= reader or not any(v in r.inputs for v in made.inputs) \
+                        or not all(v in r.inputs or pos.get(v, -1) < ri for v in made.inputs):
+                    return False
                 have = {m.output for m in r.nodes}
                 joined = sorted(r.nodes + [m for m in made.nodes if m.output not in have], key=lambda m: m.output)
-                return (r.kind == "row" and r.rows == space and ri < reader and any(v in r.inputs for v in made.inputs)
-                        and all(v in r.inputs or pos.get(v, -1) < ri for v in made.inputs)
-                        and row_reads_ok(graph, joined, space))
+                return row_reads_ok(graph, joined, space)
 
             row = next((r for r in steps if takes(r)), None)
             if row is None:
@@ -596,7 +598,7 @@ def column_sums(graph, steps):
         vars(row).update(vars(summing))
         if made is not row:
             gone.add(id(made))
-        pos[red.output] = steps.index(row)
+        pos[red.output] = at[id(row)]
         gone.add(id(st))
     return _drop_unread(graph, [st for st in steps if id(st) not in gone])
 
