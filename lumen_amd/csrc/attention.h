@@ -244,7 +244,7 @@ __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     const int nfull = full_end > 0 ? int(full_end / BN) : 0;
 
     zero_tiles(stage0, 2 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
-    zero_tiles(stage1, 2 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
+    zero_tiles(stage1, 2 * TILE, ntiles > 1 && (p.sk % BN || p.hd < D || p.hdv < D));
     if (ntiles > 0) {
         load_tile_async<D, NW>(kp, p.k_s, 0, p.sk, stage0, wave, lane, p.hd);
         load_tile_async<D, NW>(vp, p.v_s, 0, p.sk, stage0 + TILE, wave, lane, p.hdv);
