@@ -208,14 +208,15 @@ template <int NW, int D = 128> struct FwdOccupancy {
 // The two stages are arrays of their own, named by a constant in the loop below: were they halves of one array, every
 // LDS read would be taken to alias the loads just issued into the other half and wait for them (s_waitcnt vmcnt(0)
 // before the tile's first read), so that nothing overlapped. [8, 2048, 16, 128] causal 243 -> 192-203 us (679-716
-// TFLOP/s), [2, 1777, 16 / 4, 64] 43 -> 37.
-template <int D, bool F16, bool CAUSAL, int NW>
+// TFLOP/s), [2, 1777, 16 / 4, 64] 43 -> 37. ONE: halves of one array after all, for fewer registers (launch_fwd_nw).
+template <int D, bool F16, bool CAUSAL, int NW, bool ONE = false>
 __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     constexpr int QB = 32 * NW;  // queries a workgroup
     constexpr int BN = 64;
     constexpr int DS = D / 16, DT = D / 32;
     constexpr int TILE = BN * D;  // elements
-    __shared__ __align__(1024) uint16_t stage0[2 * TILE], stage1[2 * TILE];  // K, V
+    __shared__ __align__(1024) uint16_t stage0[(ONE ? 4 : 2) * TILE], apart[ONE ? 8 : 2 * TILE];  // K, V
+    uint16_t *const stage1 = ONE ? stage0 + 2 * TILE : apart;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
     const int g = lane >> 4, s16 = lane & 15;
@@ -345,9 +346,13 @@ __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
             }
         }
     };
-    for (int kt = 0; kt < ntiles; kt += 2) {
-        tile(kt, stage0, stage1);
-        if (kt + 1 < ntiles) tile(kt + 1, stage1, stage0);
+    if constexpr (ONE) {
+        for (int kt = 0; kt < ntiles; ++kt) tile(kt, stage0 + (kt & 1) * 2 * TILE, stage0 + (~kt & 1) * 2 * TILE);
+    } else {
+        for (int kt = 0; kt < ntiles; kt += 2) {
+            tile(kt, stage0, stage1);
+            if (kt + 1 < ntiles) tile(kt + 1, stage1, stage0);
+        }
     }
 
     l += __shfl_xor(l, 32, 64);
@@ -368,7 +373,7 @@ __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
 
 template <int D, bool F16, bool CAUSAL, int NW = 4, int WAVES = FwdOccupancy<NW, D>::kBlocks>
 __global__ __launch_bounds__(64 * NW, WAVES) void flash_fwd_kernel(AttnParams p) {
-    flash_fwd_body<D, F16, CAUSAL, NW>(p);
+    flash_fwd_body<D, F16, CAUSAL, NW, (NW == 4 && WAVES == 4)>(p);
 }
 
 template <bool F16>
@@ -1231,9 +1236,13 @@ inline int check_attn(const nhip_attn_desc *d, const char *what, int64_t max_hd 
 template <int D, bool F16, bool CAUSAL, int NW>
 int launch_fwd_nw(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_desc *d) {
     dim3 grid(unsigned((d->sq + 32 * NW - 1) / (32 * NW) * d->heads * d->batch));
-    if constexpr (D == 64 && CAUSAL && NW == 4) {
-        if (grid.x <= 640) {
-            hipLaunchKernelGGL((nhipk::flash_fwd_kernel<D, F16, CAUSAL, NW, 2>), grid, dim3(64 * NW), 0, s, p);
+    if constexpr (D == 64 && NW == 4) {
+        // Waves a SIMD: two where a causal launch nearly fits them (FwdOccupancy); four where a launch without a mask
+        // fits them and not three, which would run a second round for a few workgroups (us with three, four: 784
+        // workgroups of 3494 keys 161.5, 153.6; 800 of 571 34.3, 32.7; 832 of 141 18.0, 15.9; 988 of 6914 330, 323).
+        constexpr int kWaves = CAUSAL ? 2 : 4;
+        if (CAUSAL ? grid.x <= 640 : grid.x > 768 && grid.x <= 1024) {
+            hipLaunchKernelGGL((nhipk::flash_fwd_kernel<D, F16, CAUSAL, NW, kWaves>), grid, dim3(64 * NW), 0, s, p);
             return check(hipGetLastError(), "flash_fwd launch");
         }
     }

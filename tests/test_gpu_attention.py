@@ -380,3 +380,22 @@ def test_default_forward_tile_gives_the_configs_bits(hip, sq, sk, d, causal):
     for x in got[1:]:
         np.testing.assert_array_equal(x[0], got[0][0])
         np.testing.assert_array_equal(x[1], got[0][1])
+
+
+@pytest.mark.parametrize("b,sq,sk,d", [(100, 30, 200, 64), (64, 129, 67, 64), (60, 200, 513, 40), (96, 30, 200, 64),
+                                       (65, 129, 64, 64)])
+def test_forward_at_four_waves_a_simd_gives_the_other_tiles_bits(hip, b, sq, sk, d):
+    """Launches without a mask that fit four workgroups a CU and not three (config 0) share one array between the stages:
+    the bits of the 64-query workgroups (config 2), for odd and even tile counts, ragged tiles and a padded head dim; the
+    last two lie past the bounds of that range."""
+    n = 8
+    rng = np.random.default_rng(sk)
+    q, k, v = (D.bf16_bits(rng.standard_normal(s).astype(np.float32)) for s in ((b, sq, n, d), (b, sk, n, d), (b, sk, n, d)))
+    desc = attn_desc(b, sq, sk, n, n, d, False, 1.0 / math.sqrt(d))
+    dq, dk, dv, o, lse = Dev(q), Dev(k), Dev(v), Dev(nbytes=q.nbytes), Dev(nbytes=b * n * sq * 4)
+    got = []
+    for config in (0, 2):
+        desc.config = config
+        nv.call("nhip_flash_fwd", C.byref(desc), dq.ptr, dk.ptr, dv.ptr, o.ptr, lse.ptr)
+        got.append((o.get(q.shape, np.uint16), lse.get((b, n, sq), np.uint32)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
