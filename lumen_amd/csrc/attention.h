@@ -245,6 +245,7 @@ __device__ __forceinline__ void flash_fwd_body(const AttnParams &p) {
     const int nfull = full_end > 0 ? int(full_end / BN) : 0;
 
     zero_tiles(stage0, 2 * TILE, p.sk % BN || p.hd < D || p.hdv < D);
+    // one tile reads no second stage (134 shapes of up to 64 keys at head dims above 64 take 0.955 of the time with it cleared)
     zero_tiles(stage1, 2 * TILE, ntiles > 1 && (p.sk % BN || p.hd < D || p.hdv < D));
     if (ntiles > 0) {
         load_tile_async<D, NW>(kp, p.k_s, 0, p.sk, stage0, wave, lane, p.hd);
@@ -1239,7 +1240,7 @@ int launch_fwd_nw(hipStream_t s, const nhipk::AttnParams &p, const nhip_attn_des
     if constexpr (D == 64 && NW == 4) {
         // Waves a SIMD: two where a causal launch nearly fits them (FwdOccupancy); four where a launch without a mask
         // fits them and not three, which would run a second round for a few workgroups (us with three, four: 784
-        // workgroups of 3494 keys 161.5, 153.6; 800 of 571 34.3, 32.7; 832 of 141 18.0, 15.9; 988 of 6914 330, 323).
+        // workgroups of 3494 keys 153.3, 148.3; 800 of 1212 58.8, 56.5; 832 of 141 17.6, 17.1; 988 of 6914 316, 308).
         constexpr int kWaves = CAUSAL ? 2 : 4;
         if (CAUSAL ? grid.x <= 640 : grid.x > 768 && grid.x <= 1024) {
             hipLaunchKernelGGL((nhipk::flash_fwd_kernel<D, F16, CAUSAL, NW, kWaves>), grid, dim3(64 * NW), 0, s, p);
