@@ -1418,7 +1418,9 @@ class LoopKernel:
     # thread wide (16384, 8 at a time) and their sums at most SUM_REGISTERS together: wider ones spill. [R, C] norm
     # backward in us with the sums here and in reductions of their own: [256, 16384] 24, 27; [4096, 16384] 114, 260; scale
     # and shift, [4096, 12288] (48 registers) 124, 297. Past it: [256, 24576] 45, 33; scale and shift [256, 16384] 58, 44;
-    # a vocabulary head's bias, 8192 rows of 32000 1783, 1532, of 50304 (394 VGPRs spilled) 5059, 2293.
+    # a vocabulary head's bias, 8192 rows of 32000 1783, 1532, of 50304 (394 VGPRs spilled) 5059, 2293. Within it 46 of 48
+    # softmax and norm backwards of 515 to 8190 columns are faster here (0.37 to 1.01 of the time); not a softmax's over 11481
+    # rows of 515 (51, 58) and 1102 (62, 69), whose exponentials want more waves than the workgroups of a sum hold.
     SUM_THREADS = 512
     SUM_BLOCKS = 512
     SUM_FEW = 64
