@@ -1207,8 +1207,9 @@ class Plan:
         tiles (two a CU; at most one a CU takes 0.79 of a round), its 256 x 256 ones or, whole, its 64 x 64 ones (four a
         CU, one a CU 0.59) fit on the chip, each k long, and the partials written and read. Fitted to 367 shapes of 2^30 to
         2^38 multiply-adds in three layouts, each measured in 1, 2, 4 and 8 parts at its best config: the count this
-        gives is on average 0.6% slower than the fastest (at most 21%; filling the chip 2.7%, 39%; never dividing 44%).
-        [8192, 512] x [512, 2048] 28 us whole, 35 in two; [2048, 8192] x [8192, 512] 71, 54, 39, 37; [8192, 32000] x
+        gives is on average 0.6% slower than the fastest (at most 21%; filling the chip 2.7%, 39%; never dividing 44%); on
+        515 products of other layers' shapes 0.5%, at most 14%.
+        [8192, 2048] x [2048, 512] 28 us whole, 35 in two; [2048, 8192] x [8192, 512] 71, 54, 39, 37; [8192, 32000] x
         [32000, 512] 477, 328, 282."""
         def tiles(b):
             return -(-d.m // b) * -(-d.n // b) * z
